@@ -26,7 +26,11 @@
  *    arrives; the buffer it outgrew stays allocated until thq_destroy, so
  *    work already enqueued, or captured in a HIP graph, keeps valid memory.
  *    A call that grows the workspace cannot run under stream capture: warm
- *    every captured shape once beforehand.
+ *    every captured shape once beforehand.  Calls on f32 rows do not use the
+ *    shared workspace: they take scratch that the context keeps per stream
+ *    (at most 8 streams, until thq_destroy), so they stay re-entrant on
+ *    distinct streams; where that cannot be had (more streams, growth under
+ *    capture) they run the slower scalar kernel, which needs none.
  *  - W is [N, K] row-major (row n = output feature n), exactly the GGUF
  *    tensor layout QTensor::data() returns.  y[m, n] = sum_k x[m, k] * W[n, k].
  */
@@ -259,8 +263,9 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
  *              runs a bf16 MFMA GEMM on it, the engine's "dequant + bf16
  *              matmul" prefill route
  *   Q6_K under THQ_MODE_EXACT_W past 64 rows runs the exact decode GEMV in
- *   groups of 16 rows.  x f32 with M >= 2 runs an exact f32 path, and so do
- *   the remaining shapes.
+ *   groups of 16 rows.  x f32 with M >= 2 and K a multiple of 256 runs on
+ *   the f16 matrix cores, each row as two f16 planes, weights exact, no less
+ *   precise than f32 dots; the remaining shapes run an exact scalar f32 path.
  * THQ_MODE_Q8ACT instead reproduces candle's default CPU k_quants::matmul:
  * x rows are quantized as thq_quantize_act does (into the context
  * workspace), every block dot is exact in integers and scaled in f32; only
@@ -295,7 +300,8 @@ size_t thq_noalloc_scratch_bytes(void);
  * (gate_up = 1) call of M rows would take, on the host, and returns the
  * context workspace bytes it needs (0 for routes with no scratch); no device
  * work.  thq_reserve grows the context workspace to at least
- * workspace_bytes and the context's zeroed split-K arrival counters to at
+ * workspace_bytes, sets aside as much for the next stream that makes f32
+ * calls (a capture stream, which cannot allocate), and the context's zeroed split-K arrival counters to at
  * least `counters` entries (one per 32-row output tile of the widest
  * weight, and 32 per row of a top-k call, at most 65536), synchronously (hipMalloc, hipMemset, device synchronize); calls
  * whose needs fit then allocate nothing.  thq_workspace_bytes returns the

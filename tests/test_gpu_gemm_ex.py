@@ -1,0 +1,153 @@
+"""f32 activations on the f16 matrix cores (k_gemm_ex.hip): every format,
+plain and gate/up, against the f64 product with the library's f32
+dequantization (pinned bit-exact elsewhere).
+
+Bound: relative error of the whole result (2-norm) <= 2e-7.  The scalar f32
+kernel it replaces measures 1.18e-7 .. 1.37e-7 over K = 1024 .. 17408, this
+one 0.8e-7 .. 1.33e-7; the reference's own f32-rounded weights add about 4e-8.
+Covered: the stacked form's edge (16 / 17 rows), whole and partial row groups,
+ragged outputs, one chunk and several K splits, bf16 output, rows of very
+large, very small and non-finite values, growth under capture (the general
+kernel runs), replays of a captured call, and calls on two streams.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import activations, q6k_bytes, rand_qlin_fast, weight_bytes
+
+pytestmark = pytest.mark.gpu
+
+thq = pytest.importorskip("thq")
+FORMATS = ["q8_0", "q4_k", "q6_k", "affine"]
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.init()
+    yield
+    torch.cuda.synchronize()
+
+
+def weight(fmt, n, k, ctx=None):
+    if fmt == "affine":
+        wq, sb = rand_qlin_fast(n, k, seed=n + k)
+        return thq.QTensor.from_affine(wq, sb, n, k, ctx=ctx)
+    if fmt == "q6_k":
+        return thq.QTensor.from_gguf_bytes(thq.Q6_K, q6k_bytes(n, k, seed=3), n, k, ctx=ctx)
+    qt = O.Q8_0 if fmt == "q8_0" else O.Q4_K
+    return thq.QTensor.from_gguf_bytes(qt, weight_bytes(qt, n, k, seed=3), n, k, ctx=ctx)
+
+
+def rows(m, k, seed=0):
+    return torch.from_numpy(activations(m, k, seed=seed)).cuda()
+
+
+def rel(y, ref):
+    return float((y.double() - ref).norm() / ref.norm())
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(2, 40, 256), (16, 300, 1792), (17, 512, 1024), (33, 257, 2048), (70, 1000, 4096),
+                                   (3, 96, 17408)])
+def test_rows_match_f64(fmt, m, n, k):
+    w, x = weight(fmt, n, k), rows(m, k)
+    ref = x.double() @ w.dequantize().double().T
+    assert rel(thq.matmul(w, x, torch.float32), ref) <= 2e-7
+    assert rel(thq.matmul(w, x, torch.bfloat16), ref) <= 2e-3  # bf16 rounding of the result: 2^-9 / sqrt(3)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,h,k", [(5, 96, 512), (40, 200, 1792)])
+def test_gate_up(fmt, m, h, k, monkeypatch):
+    w, x = weight(fmt, 2 * h, k), rows(m, k, seed=4)
+    y = thq.gate_up_silu(w, x, torch.float32)
+    monkeypatch.setenv("THQ_GEMM_EX", "0")
+    ref = thq.gate_up_silu(w, x, torch.float32)
+    # both round their gate and up sums to bf16: equal but where a sum lies between two neighbours
+    assert rel(y, ref.double()) <= 1e-3
+    assert float((y != ref).float().mean()) <= 0.02
+
+
+def test_q6k_single_row():
+    w, x = weight("q6_k", 130, 512), rows(1, 512)
+    assert rel(thq.matmul(w, x, torch.float32), x.double() @ w.dequantize().double().T) <= 2e-7
+
+
+@pytest.mark.parametrize("m", [6, 40])
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_extreme_rows(fmt, m):
+    n, k = 64, 512
+    w, x = weight(fmt, n, k), rows(m, k, seed=7)
+    x[0] *= 1e30
+    x[1] *= 1e-33
+    x[2] = 0.0
+    x[3, 5] = 3e4 * x[3].abs().max()  # one outlier: the rest still carries
+    ref = x.double() @ w.dequantize().double().T
+    y = thq.matmul(w, x, torch.float32)
+    for i in (0, 1, 3, 4):
+        assert rel(y[i], ref[i]) <= 3e-7, i
+    assert not y[2].any()
+    x[1, 9] = float("inf")
+    x[4, 300] = float("nan")
+    z = thq.matmul(w, x, torch.float32)
+    wd = w.dequantize()
+    assert z[4].isnan().all()
+    assert torch.equal(z[1][wd[:, 9] != 0], torch.sign(wd[:, 9][wd[:, 9] != 0]) * float("inf"))
+    keep = [i for i in range(m) if i not in (1, 4)]
+    assert torch.equal(z[keep], y[keep])
+
+
+def test_capture_without_scratch_and_replay():
+    """A stream whose scratch would have to grow under capture takes the general kernel; one that has it, its own."""
+    ctx = thq.Context(0)
+    w, x = weight("q4_k", 256, 1024, ctx), rows(5, 1024)
+    ref = x.double() @ w.dequantize().double().T
+    for warm in (False, True):
+        s = torch.cuda.Stream()
+        out = torch.empty((5, 256), device="cuda")
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            if warm:
+                thq.matmul(w, x, out=out)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                thq.matmul(w, x, out=out)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            torch.randn(64, 64, device="cuda") @ torch.randn(64, 64, device="cuda")
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert rel(out, ref) <= 2e-7
+
+
+def test_two_streams():
+    """f32 calls of one context on two streams do not share scratch."""
+    w = weight("q4_k", 2048, 1024)
+    xs = [rows(40, 1024, seed=20 + i) for i in range(2)]
+    ref = [thq.matmul(w, x, torch.float32) for x in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    out = [[], []]
+    for _ in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                out[i].append(thq.matmul(w, xs[i], torch.float32))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(y, ref[i]) for y in out[i])
+
+
+def test_many_rows_in_chunks():
+    """Scratch past the cap: row chunks, each row's bits as in a call of its own chunk."""
+    n, k, m = 65536, 2048, 1100
+    w, x = weight("affine", n, k), rows(m, k, seed=9)
+    assert thq.call_scratch_bytes(w, m, x_dtype=torch.float32) <= 512 << 20
+    y = thq.matmul(w, x, torch.float32)
+    pick = np.r_[0, 511, 512, 1023, 1024, 1099]
+    ref = x[pick].double() @ w.dequantize().double().T
+    assert rel(y[pick], ref) <= 2e-7

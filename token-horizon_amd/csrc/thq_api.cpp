@@ -30,6 +30,16 @@
 constexpr size_t THQ_NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[THQ_NOALLOC_SCRATCH_BYTES];
 
+// one stream's own scratch (open: made by thq_reserve, taken by the first stream that asks)
+struct thq_side {
+    hipStream_t s = nullptr;
+    bool open = false;
+    void* p = nullptr;
+    size_t bytes = 0;
+};
+
+constexpr size_t SIDE_MAX = 8;
+
 struct thq_ctx {
     int device = 0;
     void* scratch = nullptr;  // this device's copy of `scratch` (thq_init)
@@ -48,6 +58,9 @@ struct thq_ctx {
     // zero between launches; grown like the workspace
     uint32_t* tile_cnt = nullptr;
     size_t tile_cnt_n = 0;
+    // scratch of the routes that replaced scratch-free ones (side_scratch)
+    thq_side side[SIDE_MAX];
+    size_t nside = 0;
 };
 
 struct thq_weight {
@@ -206,6 +219,47 @@ uint32_t* tile_counters(thq_ctx* ctx, int64_t n) {
     return p;
 }
 
+// Scratch for f32 calls, which use no shared workspace: one buffer per stream, so that such calls
+// on distinct streams stay independent of each other and of the shared
+// workspace (caller holds ctx->mu).  At most SIDE_MAX streams, each buffer
+// kept until thq_destroy and grown like the workspace; null when it cannot be
+// had (too many streams, growth under stream capture, out of memory): the
+// caller then takes a route without it.
+void* side_scratch(thq_ctx* ctx, hipStream_t s, size_t bytes) {
+    thq_side* at = nullptr;
+    thq_side* const end = ctx->side + ctx->nside;
+    for (thq_side* e = ctx->side; e != end; ++e)
+        if (!e->open && e->s == s) at = e;
+    if (at && at->bytes >= bytes) return at->p;
+    for (thq_side* e = ctx->side; !at && e != end; ++e)
+        if (e->open && e->bytes >= bytes) {
+            e->open = false;
+            e->s = s;
+            return e->p;
+        }
+    if (!at && ctx->nside >= SIDE_MAX) return nullptr;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    size_t want = bytes + (bytes >> 3);
+    if (at && want < 2 * at->bytes) want = 2 * at->bytes;
+    void* p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (at) {
+        ctx->retired.push_back(at->p);
+        at->p = p;
+        at->bytes = want;
+    } else {
+        ctx->side[ctx->nside++] = thq_side{s, false, p, want};
+    }
+    return p;
+}
+
 struct DeviceGuard {
     int prev = -1;
     explicit DeviceGuard(int dev) {
@@ -266,6 +320,7 @@ struct Call {
     thq::AmaxOut* am;
     size_t scratch_cap = SIZE_MAX;  // routes needing more scratch are not planned
     bool counters = true;           // the caller can supply zeroed arrival counters
+    bool ex = true;                 // k_gemm_ex may be planned (its scratch can be had)
 };
 
 // an environment switch set to "0" (read on every call)
@@ -313,7 +368,7 @@ int check_call(const Call& c) {
 
 // The kernels a call runs, and the device scratch (split-K partials or the
 // quantized activation planes) they use, known before anything launches.
-enum class Kind { NONE, Q8ACT, Q8ACT_TILE, GEMV1, ROWS, GEMV_TILE, GEMV_MFMA, GEMV_MFMA_GROUPS, WIDE, GEMM, GEMM_DQ, GEMM_FQ, GEMM_RQ, GEMM_MID, GENERIC };
+enum class Kind { NONE, Q8ACT, Q8ACT_TILE, GEMV1, ROWS, GEMV_TILE, GEMV_MFMA, GEMV_MFMA_GROUPS, WIDE, GEMM, GEMM_DQ, GEMM_FQ, GEMM_RQ, GEMM_MID, GEMM_EX, GENERIC };
 struct Route {
     Kind kind = Kind::NONE;
     thq::GemvPlan gp;
@@ -324,6 +379,8 @@ struct Route {
     thq::FqPlan fq;
     thq::RqPlan rq;
     thq::MidPlan mp;
+    thq::ExPlan ep, ep_last;  // GEMM_EX: row chunks of ex_rows, and the last, partial one
+    int ex_rows = 0;
     bool exact = false;
     size_t scratch = 0;
 };
@@ -336,6 +393,35 @@ thq::TilePlan q8act_tile_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m
     static const bool on = !env_flag_off("THQ_Q8ACT_TILE");
     if (!on || !w->tq || w->qtype != THQ_Q4_K || m < 2 || m > 8) return thq::TilePlan{};
     return thq::plan_gemv_tile(m, w->N, w->K, gu, ctx->cus);
+}
+
+// f32 rows: k_gemm_ex (every format, K in whole chunks) in row chunks whose
+// scratch (activation planes, split partials) stays within EX_MAX_MB and the
+// caller's cap, wherever the scalar generic kernel ran before: from 2 rows (Q6_K
+// from 1).  Both sides at M = 5 / 300: k_gemm_ex.hip.  THQ_GEMM_EX=0 turns it off.
+constexpr size_t EX_MAX_MB = 512;
+bool plan_ex(const Call& c, Route& r) {
+    if (!c.ex || c.am || !aligned16(c.x) || env_flag_off("THQ_GEMM_EX")) return false;
+    const thq_weight* w = c.w;
+    const int qt = view(w).qtype;
+    const size_t cap = std::min(c.scratch_cap, EX_MAX_MB << 20);
+    int64_t rows = c.m;
+    thq::ExPlan p = thq::plan_gemm_ex(qt, rows, w->N, w->K, c.gu, c.ctx->cus);
+    while ((p.groups == 0 || p.workspace_bytes > cap) && rows > 64) {
+        rows = std::max<int64_t>(64, rows / 2 / 64 * 64);
+        p = thq::plan_gemm_ex(qt, rows, w->N, w->K, c.gu, c.ctx->cus);
+    }
+    if (p.groups == 0 || p.workspace_bytes > cap) return false;
+    r.ep = r.ep_last = p;
+    r.ex_rows = (int)rows;
+    r.scratch = p.workspace_bytes;
+    if (c.m % rows) {
+        r.ep_last = thq::plan_gemm_ex(qt, c.m % rows, w->N, w->K, c.gu, c.ctx->cus);
+        if (r.ep_last.groups == 0 || r.ep_last.workspace_bytes > cap) return false;
+        r.scratch = std::max(r.scratch, r.ep_last.workspace_bytes);
+    }
+    r.kind = Kind::GEMM_EX;
+    return true;
 }
 
 // Routing by rows, as QLin::linear_ps (engine/src/qwen35.rs:398-617).  A
@@ -459,6 +545,7 @@ Route plan_route(const Call& c) {
         }
     } else if (c.am) {
         // no fused epilogue
+    } else if (xf32 && plan_ex(c, r)) {
     } else if (!xf32 && aligned16(c.x) && w->K % 64 == 0 &&  // the GEMMs step K in 64-wide tiles
                // gate/up rows of < 256 outputs: the rounded-weight tile's error, seen
                // through silu(g)*u, is not averaged down by the row norm (the exact
@@ -657,6 +744,18 @@ int exec_route(const Call& c, const Route& r, void* scratch, uint32_t* cnt = nul
             e = dequant_any(w, scratch, true, c.s);
             if (e == hipSuccess) e = thq::launch_gemm_b16(c.x, scratch, c.y, yf32, m, (int)w->N, (int)w->K, c.s);
             break;
+        case Kind::GEMM_EX: {
+            // chunks run in stream order, so they share the scratch
+            const size_t yrow = (size_t)nout * (yf32 ? 4 : 2);
+            for (int64_t r0 = 0; r0 < m && e == hipSuccess; r0 += r.ex_rows) {
+                const int mm = (int)std::min<int64_t>(m - r0, r.ex_rows);
+                e = thq::launch_gemm_ex(mm == r.ex_rows ? r.ep : r.ep_last, v,
+                                        static_cast<const float*>(c.x) + r0 * w->K,
+                                        static_cast<char*>(c.y) + r0 * yrow, yf32, c.gu, mm, nout, up_off, scratch,
+                                        c.s);
+            }
+            break;
+        }
         case Kind::GENERIC: e = thq::launch_generic(v, c.x, xf32, c.y, yf32, c.gu, m, nout, up_off, c.s); break;
     }
     if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
@@ -669,9 +768,16 @@ int run_matmul(const Call& c) {
     if (rc || c.m == 0) return rc;
     if (c.am) c.am->nb = 0;
     DeviceGuard g(c.ctx->device);
-    const Route r = plan_route(c);
+    Route r = plan_route(c);
     if (r.kind == Kind::NONE) return THQ_OK;
     std::lock_guard<std::mutex> lk(c.ctx->mu);
+    if (r.kind == Kind::GEMM_EX) {
+        void* p = side_scratch(c.ctx, c.s, r.scratch);
+        if (p) return exec_route(c, r, p);
+        Call d = c;
+        d.ex = false;
+        r = plan_route(d);
+    }
     if (r.scratch) {
         rc = ensure_ws(c.ctx, r.scratch);
         if (rc) return rc;
@@ -719,12 +825,13 @@ int thq_init(int device, thq_ctx** out) {
 
 void thq_destroy(thq_ctx* ctx) {
     if (!ctx) return;
-    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || !ctx->retired.empty()) {
+    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || ctx->nside || !ctx->retired.empty()) {
         DeviceGuard g(ctx->device);
         (void)hipDeviceSynchronize();
         if (ctx->ws) (void)hipFree(ctx->ws);
         if (ctx->emit_cnt) (void)hipFree(ctx->emit_cnt);
         if (ctx->tile_cnt) (void)hipFree(ctx->tile_cnt);
+        for (size_t i = 0; i < ctx->nside; ++i) (void)hipFree(ctx->side[i].p);
         for (void* p : ctx->retired) (void)hipFree(p);
     }
     delete ctx;
@@ -1268,6 +1375,19 @@ int thq_reserve(thq_ctx* ctx, size_t workspace_bytes, int64_t counters) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     int rc = ensure_ws(ctx, workspace_bytes);
     if (rc) return rc;
+    if (workspace_bytes) {
+        // the same for the calls with a scratch of their own: a buffer that the
+        // next stream without one takes (a capture stream, which cannot allocate)
+        bool have = false;
+        for (size_t i = 0; i < ctx->nside; ++i) have |= ctx->side[i].open && ctx->side[i].bytes >= workspace_bytes;
+        if (!have && ctx->nside < SIDE_MAX) {
+            void* p = nullptr;
+            hipError_t e = hipMalloc(&p, workspace_bytes);
+            if (e != hipSuccess)
+                return fail(THQ_ENOMEM, "workspace hipMalloc(%zu): %s", workspace_bytes, hipGetErrorString(e));
+            ctx->side[ctx->nside++] = thq_side{nullptr, true, p, workspace_bytes};
+        }
+    }
     if (counters > 0 && !tile_counters(ctx, counters))
         return fail(THQ_ENOMEM, "arrival counters (%lld entries) could not be allocated", (long long)counters);
     HIP_TRY(hipDeviceSynchronize());

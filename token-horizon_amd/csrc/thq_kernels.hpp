@@ -169,6 +169,18 @@ bool gemm_rq_supported(int qtype, int64_t M, int64_t N_rows, int64_t K, bool gu)
 RqPlan plan_gemm_rq(int64_t M, int64_t N_rows, int64_t K, bool gu, int cus);
 hipError_t launch_gemm_rq(const RqPlan& p, bool affine, const uint8_t* wq, const void* x, void* y, bool yf32, bool gu,
                           int M, int64_t N_rows, int K, float* ws, uint32_t* cnt, hipStream_t s);
+// f32 rows (16-B aligned) over every format, K % 256 == 0, plain or gate/up,
+// on row-scaled f16 activation planes (k_gemm_ex.hip); the workspace holds
+// the planes, then the split partials
+struct ExPlan {
+    bool stacked = false;     // up to 16 rows, both planes in one operand
+    int groups = 0;           // row groups (0: unsupported)
+    int splits = 0, cps = 0;  // K splits, 256-wide chunks per split
+    size_t workspace_bytes = 0;
+};
+ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus);
+hipError_t launch_gemm_ex(const ExPlan& p, const WeightView& w, const float* x, void* y, bool yf32, bool gu, int M,
+                          int64_t nout, int64_t up_off, void* ws, hipStream_t s);
 // exact generic kernel, any M, scalar activation loads
 hipError_t launch_generic(const WeightView& w, const void* x, bool xf32, void* y, bool yf32, bool gu, int M,
                           int64_t nout, int64_t up_off, hipStream_t s);
