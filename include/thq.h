@@ -27,7 +27,8 @@
  *    work already enqueued, or captured in a HIP graph, keeps valid memory.
  *    A call that grows the workspace cannot run under stream capture: warm
  *    every captured shape once beforehand.  Calls on f32 rows do not use the
- *    shared workspace: they take scratch that the context keeps per stream
+ *    shared workspace: they (and the split sums of thq_matmul_q8act from 9 rows)
+ *    take scratch that the context keeps per stream
  *    (at most 8 streams, until thq_destroy), so they stay re-entrant on
  *    distinct streams; where that cannot be had (more streams, growth under
  *    capture) they run the slower scalar kernel, which needs none.
@@ -270,7 +271,8 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
  * x rows are quantized as thq_quantize_act does (into the context
  * workspace), every block dot is exact in integers and scaled in f32; only
  * the f32 summation order over blocks differs from candle's (2..8 rows of
- * a Q4_K weight with a tile plane take int8 matrix-core dots over it).  Any
+ * a Q4_K weight with a tile plane, and larger calls from 9 rows with K a
+ * multiple of 256, take int8 matrix-core dots).  Any
  * M; x must be 16-byte aligned (THQ_EALIGN otherwise).
  * Inputs: x_dev [M, K] of x_type, y_dev [M, N] of y_type, both contiguous.
  * M == 0 is a no-op.  Errors: THQ_ESHAPE for K mismatch, THQ_EINVAL for

@@ -1,0 +1,106 @@
+"""THQ_MODE_Q8ACT over many rows on the int8 matrix cores (k_q8act_gemm.hip)
+against the row-tile kernels (THQ_Q8ACT_GEMM=0, themselves pinned to the
+oracle): the same exact block integers, so only the f32 order differs: relative
+2-norm <= 4e-7 (the row-tile kernels are up to 2.1e-7 from 64-bit sums, this
+one up to 0.8e-7).  Covered: row-group edges, ragged outputs, one chunk and K
+splits, extreme quants (every product at its largest: the two int8 planes, the
+minimum's sums), gate/up, prepared buffers, the emitted operand, and the rule.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from helpers import activations, weight_bytes
+
+pytestmark = pytest.mark.gpu
+
+thq = pytest.importorskip("thq")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    torch.cuda.init()
+    yield
+    torch.cuda.synchronize()
+
+
+def rel(y, ref):
+    return float((y.double() - ref.double()).norm() / ref.double().norm())
+
+
+def both(monkeypatch, f):
+    out = []
+    for v in ("0", "1"):
+        monkeypatch.setenv("THQ_Q8ACT_GEMM", v)
+        out.append(f())
+    return out
+
+
+@pytest.mark.parametrize("qt", [O.Q4_K, O.Q8_0])
+@pytest.mark.parametrize("m,n,k", [(1, 40, 256), (31, 300, 1792), (33, 512, 1024), (64, 257, 2048), (70, 1000, 4096),
+                                   (9, 96, 17408)])
+def test_matches_row_tiles(qt, m, n, k, monkeypatch):
+    w = thq.QTensor.from_gguf_bytes(qt, weight_bytes(qt, n, k, seed=5), n, k)
+    x = torch.from_numpy(activations(m, k, seed=6)).cuda()
+    ref, y = both(monkeypatch, lambda: thq.matmul(w, x, torch.float32, thq.MODE_Q8ACT))
+    assert rel(y, ref) <= 4e-7
+    q = thq.Q8Act(x, thq.Q8_K if qt == O.Q4_K else thq.Q8_0)
+    assert torch.equal(q.matmul(w, torch.float32), y)
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_largest_integers(sign, monkeypatch):
+    """All nibbles 15, all scales and minima 63, all quants -128 (or 127): the largest sums the planes can reach."""
+    n, k, m = 64, 512, 40
+    blk = np.zeros((n, k // 256, 144), np.uint8)
+    blk[:, :, 0:4] = np.array([1.0, 0.5], np.float16).view(np.uint8)
+    blk[:, :, 4:] = 0xFF
+    w = thq.QTensor.from_gguf_bytes(O.Q4_K, blk.reshape(n, -1), n, k)
+    x = torch.full((m, k), sign, device="cuda")
+    x[:, ::256] = -sign * 1.001  # the block's largest: -128 of the other sign
+    ref, y = both(monkeypatch, lambda: thq.matmul(w, x, torch.float32, thq.MODE_Q8ACT))
+    assert rel(y, ref) <= 4e-7
+
+
+@pytest.mark.parametrize("qt", [O.Q4_K, O.Q8_0])
+def test_gate_up_and_emit(qt, monkeypatch):
+    h, k, m = 256, 1024, 64  # whole 256-B planes: the buffers hold no padding
+    w = thq.QTensor.from_gguf_bytes(qt, weight_bytes(qt, 2 * h, k, seed=8), 2 * h, k)
+    x = torch.from_numpy(activations(m, k, seed=9)).cuda()
+    ref, y = both(monkeypatch, lambda: thq.gate_up_silu(w, x, torch.float32, thq.MODE_Q8ACT))
+    assert rel(y, ref) <= 1e-3 and float((y != ref).float().mean()) <= 0.02  # sums round to bf16 first
+    if qt == O.Q4_K:
+        z, nxt = thq.Q8Act(x, thq.Q8_K).gate_up_silu_emit(w, torch.float32)
+        assert torch.equal(z, y)
+        assert torch.equal(nxt.buf, thq.Q8Act(y, thq.Q8_K).buf)
+
+
+def test_rule_and_capture():
+    ctx = thq.Context(0)
+    n, k, m = 4096, 1024, 96  # large enough for the int8 GEMM, K splits among them
+    w = thq.QTensor.from_gguf_bytes(O.Q4_K, weight_bytes(O.Q4_K, n, k, seed=5), n, k, ctx=ctx)
+    x = torch.from_numpy(activations(m, k, seed=6)).cuda()
+    q = thq.Q8Act(x, thq.Q8_K, ctx=ctx)
+    s = torch.cuda.Stream()
+    out = []
+    with torch.cuda.stream(s):
+        s.wait_stream(torch.cuda.default_stream())
+        for warm in (False, True):  # without scratch of its own a captured call runs the row-tile kernels
+            if warm:
+                ref = q.matmul(w, torch.float32)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                y = q.matmul(w, torch.float32)
+            out.append((g, y))
+    for g, y in out:
+        for _ in range(3):
+            y.fill_(float("nan"))
+            torch.randn(64, 64, device="cuda") @ torch.randn(64, 64, device="cuda")
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert rel(y, ref) <= 4e-7
+    assert torch.equal(out[1][1], ref)

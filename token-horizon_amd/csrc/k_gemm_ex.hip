@@ -503,9 +503,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
     __syncthreads();
     // step c (buffer b): chunk c + 1's copies go out first (buffer b ^ 1, read
     // by no wave since the last barrier); each half's weights are loaded again
-    // for chunk c + 1 as soon as it is consumed; the copies and the first
-    // half's loads are waited for before the second half's go out, which stay
-    // in flight across the barrier.  Past the range they repeat the last chunk.
+    // for chunk c + 1 as soon as it is consumed and stay in flight across the
+    // barrier: loads complete in order and the first half's and the header's
+    // are ten or more instructions behind the copies, so vmcnt(10) waits for
+    // the copies only.  Past the range they repeat the last chunk.
     for (int c = cb; c < ce; ++c) {
         const int b = (c - cb) & 1;
         float d[2], dm[2];
@@ -539,12 +540,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
         if constexpr (QT == 12) offsets(Hc, d, dm, As);
         sstore(sn, b ^ 1);
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         wload(R1, last(c + 1), 1);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     }
 
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land in LDS after the block ends
     // epilogue: acc[t][e] is operand row 8 (e / 4) + 4 g + e % 4
     auto put = [&](int m, int t, float v, float vu) {
         if constexpr (OUT == 0) {
@@ -665,8 +667,7 @@ hipError_t run_ex(const ExPlan& p, const WeightView& w, const float* x, const Ex
         THQ_EX(0, (void*)b.part);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        return yf32 ? ex_reduce<GU, float>(b.part, static_cast<float*>(y), M, nout, up_off, w.N, p.splits, s)
-                    : ex_reduce<GU, bf16_t>(b.part, static_cast<bf16_t*>(y), M, nout, up_off, w.N, p.splits, s);
+        return launch_ex_reduce(b.part, y, yf32, GU, M, nout, up_off, w.N, p.splits, s);
     }
     if (yf32)
         THQ_EX(1, y);
@@ -677,6 +678,15 @@ hipError_t run_ex(const ExPlan& p, const WeightView& w, const float* x, const Ex
 }
 
 }  // namespace
+
+hipError_t launch_ex_reduce(const float* P, void* y, bool yf32, bool gu, int M, int64_t nout, int64_t up_off,
+                            int64_t ld, int S, hipStream_t s) {
+    if (yf32)
+        return gu ? ex_reduce<true, float>(P, static_cast<float*>(y), M, nout, up_off, ld, S, s)
+                  : ex_reduce<false, float>(P, static_cast<float*>(y), M, nout, up_off, ld, S, s);
+    return gu ? ex_reduce<true, bf16_t>(P, static_cast<bf16_t*>(y), M, nout, up_off, ld, S, s)
+              : ex_reduce<false, bf16_t>(P, static_cast<bf16_t*>(y), M, nout, up_off, ld, S, s);
+}
 
 ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus) {
     ExPlan p;

@@ -784,6 +784,12 @@ hipError_t launch_q8act_dot_tile(const TilePlan& p, const WeightView& w, const u
     return launch_q8act_tile(p, w, tiles, a.xq, a.xd, a.xb, y, yf32, gu, M, ws, cnt, s);
 }
 
+hipError_t launch_q8act_dot_gemm(const QgPlan& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
+                                 int M, int64_t nout, int64_t up_off, float* ws, hipStream_t s) {
+    const ActPlanes a = act_planes(w.qtype, const_cast<void*>(planes), M, w.K);
+    return launch_q8act_gemm(p, w, a.xq, a.xd, a.xb, y, yf32, gu, M, nout, up_off, ws, s);
+}
+
 hipError_t launch_q8act_tiled(const TilePlan& p, const WeightView& w, const uint8_t* tiles, const void* x, bool xf32,
                               void* y, bool yf32, bool gu, int M, void* planes, float* ws, uint32_t* cnt,
                               hipStream_t s) {

@@ -368,7 +368,7 @@ int check_call(const Call& c) {
 
 // The kernels a call runs, and the device scratch (split-K partials or the
 // quantized activation planes) they use, known before anything launches.
-enum class Kind { NONE, Q8ACT, Q8ACT_TILE, GEMV1, ROWS, GEMV_TILE, GEMV_MFMA, GEMV_MFMA_GROUPS, WIDE, GEMM, GEMM_DQ, GEMM_FQ, GEMM_RQ, GEMM_MID, GEMM_EX, GENERIC };
+enum class Kind { NONE, Q8ACT, Q8ACT_TILE, Q8ACT_GEMM, GEMV1, ROWS, GEMV_TILE, GEMV_MFMA, GEMV_MFMA_GROUPS, WIDE, GEMM, GEMM_DQ, GEMM_FQ, GEMM_RQ, GEMM_MID, GEMM_EX, GENERIC };
 struct Route {
     Kind kind = Kind::NONE;
     thq::GemvPlan gp;
@@ -381,6 +381,7 @@ struct Route {
     thq::MidPlan mp;
     thq::ExPlan ep, ep_last;  // GEMM_EX: row chunks of ex_rows, and the last, partial one
     int ex_rows = 0;
+    thq::QgPlan qg;
     bool exact = false;
     size_t scratch = 0;
 };
@@ -393,6 +394,26 @@ thq::TilePlan q8act_tile_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m
     static const bool on = !env_flag_off("THQ_Q8ACT_TILE");
     if (!on || !w->tq || w->qtype != THQ_Q4_K || m < 2 || m > 8) return thq::TilePlan{};
     return thq::plan_gemv_tile(m, w->N, w->K, gu, ctx->cus);
+}
+
+// THQ_MODE_Q8ACT rows without a tile kernel on the int8 matrix cores
+// (k_q8act_gemm) from 9 rows, where the call is large enough to pay for its
+// K splits (row-tile kernels / it, us; Q4_K 12288 x 4096 at M = 9 / 64 / 256:
+// 33.6 / 108.9 / 408 against 20.5 / 30.6 / 69; 4096 x 12288 at M = 9 / 16: 23.0
+// / 31.0 against 26.0 / 27.0; 4096 x 4096 at M = 16 / 24: 16.8 / 22.0 against
+// 17.8 / 18.6; 3072 x 1024 at M = 32 / 48: 17.3 / 24.0 against 17.5 / 17.2.
+// Q8_0, whose row-tile kernel is on int8 MFMAs already: 12288 x 4096 at M =
+// 16 / 24: 18.0 / 26.9 against 20.7 / 21.8; 4096 x 12288 at M = 9: 28.0 / 24.5;
+// 4096 x 4096 at M = 64 / 128: 16.9 / 29.4 against 19.9 / 25.0).
+// THQ_Q8ACT_GEMM: 0 never, 1 wherever supported (tests), unset: that rule.
+constexpr size_t QG_MAX_MB = 2048;  // of split partials
+thq::QgPlan q8act_gemm_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m, bool gu) {
+    const char* e = getenv("THQ_Q8ACT_GEMM");
+    const double size = (double)m * (double)w->N * (double)w->K;
+    const double least = w->qtype == THQ_Q8_0 ? (w->N < w->K ? 4.5e8 : 1.3e9) : (m >= 48 ? 1.5e8 : w->N < w->K ? 8e8 : 3e8);
+    if (e && *e ? *e != '1' : m < 9 || size < least) return thq::QgPlan{};
+    const thq::QgPlan p = thq::plan_q8act_gemm(view(w).qtype, m, w->N, w->K, gu, ctx->cus);
+    return p.workspace_bytes <= QG_MAX_MB << 20 ? p : thq::QgPlan{};
 }
 
 // f32 rows: k_gemm_ex (every format, K in whole chunks) in row chunks whose
@@ -444,6 +465,14 @@ Route plan_route(const Call& c) {
             r.kind = Kind::Q8ACT_TILE;
             r.tp = tp;
             r.scratch = align_up(r.scratch, 256) + tp.workspace_bytes;
+            return r;
+        }
+        const thq::QgPlan qg = q8act_gemm_plan(c.ctx, w, m, c.gu);
+        const size_t need = align_up(r.scratch, 256) + qg.workspace_bytes;
+        if (qg.groups > 0 && need <= c.scratch_cap) {
+            r.kind = Kind::Q8ACT_GEMM;
+            r.qg = qg;
+            r.scratch = need;
         }
         return r;
     }
@@ -698,6 +727,14 @@ int exec_route(const Call& c, const Route& r, void* scratch, uint32_t* cnt = nul
             char* planes = static_cast<char*>(scratch);
             float* part = reinterpret_cast<float*>(planes + align_up(thq::q8act_workspace_bytes(w->qtype, m, w->K), 256));
             e = thq::launch_q8act_tiled(r.tp, v, w->tq, c.x, xf32, c.y, yf32, c.gu, m, planes, part, cnt, c.s);
+            break;
+        }
+        case Kind::Q8ACT_GEMM: {
+            char* planes = static_cast<char*>(scratch);
+            float* part = reinterpret_cast<float*>(planes + align_up(thq::q8act_workspace_bytes(w->qtype, m, w->K), 256));
+            e = thq::launch_q8act_prepare(w->qtype, c.x, xf32, m, w->K, planes, c.s);
+            if (e == hipSuccess)
+                e = thq::launch_q8act_dot_gemm(r.qg, v, planes, c.y, yf32, c.gu, m, nout, up_off, part, c.s);
             break;
         }
         case Kind::GEMV1: e = thq::launch_gemv1(v, c.x, xf32, c.y, yf32, c.gu, nout, up_off, c.s, c.am); break;
@@ -1253,8 +1290,20 @@ int run_q8act_dot(thq_ctx* ctx, const thq_weight* w, thq_dtype dot_type, const v
         e = thq::launch_q8act_dot_tile(tp, view(w), w->tq, buf, y, yt == THQ_ACT_F32, gu, (int)m,
                                        static_cast<float*>(ctx->ws), cnt, static_cast<hipStream_t>(stream));
     } else {
-        e = thq::launch_q8act_dot(view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0,
-                                  static_cast<hipStream_t>(stream));
+        const hipStream_t s = static_cast<hipStream_t>(stream);
+        const thq::QgPlan qg = q8act_gemm_plan(ctx, w, m, gu);
+        void* part = nullptr;
+        bool ok = qg.groups > 0;
+        if (ok && qg.splits > 1) {
+            std::lock_guard<std::mutex> lk(ctx->mu);
+            part = side_scratch(ctx, s, qg.workspace_bytes);
+            ok = part != nullptr;
+        }
+        if (ok)
+            e = thq::launch_q8act_dot_gemm(qg, view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0,
+                                           static_cast<float*>(part), s);
+        else
+            e = thq::launch_q8act_dot(view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0, s);
     }
     if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
     return THQ_OK;
@@ -1297,6 +1346,17 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
         }
         hipError_t e = thq::launch_q8act_dot_tile(tp, view(fused), fused->tq, buf_dev, y_dev, y_type == THQ_ACT_F32,
                                                   true, (int)m, static_cast<float*>(ctx->ws), cnt, s);
+        if (e == hipSuccess)
+            e = thq::launch_q8act_prepare(12, y_dev, y_type == THQ_ACT_F32, m, nout, next_buf_dev, s);
+        if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
+        return THQ_OK;
+    }
+    const thq::QgPlan qg = q8act_gemm_plan(ctx, fused, m, true);
+    void* part = qg.groups > 0 && qg.splits > 1 ? side_scratch(ctx, s, qg.workspace_bytes) : nullptr;
+    if (qg.groups > 0 && (qg.splits == 1 || part)) {
+        // many rows: the same two launches on the int8 matrix cores
+        hipError_t e = thq::launch_q8act_dot_gemm(qg, view(fused), buf_dev, y_dev, y_type == THQ_ACT_F32, true, (int)m,
+                                                  nout, nout, static_cast<float*>(part), s);
         if (e == hipSuccess)
             e = thq::launch_q8act_prepare(12, y_dev, y_type == THQ_ACT_F32, m, nout, next_buf_dev, s);
         if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));

@@ -181,6 +181,9 @@ struct ExPlan {
 ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus);
 hipError_t launch_gemm_ex(const ExPlan& p, const WeightView& w, const float* x, void* y, bool yf32, bool gu, int M,
                           int64_t nout, int64_t up_off, void* ws, hipStream_t s);
+// K-split partials P [S][M][ld] summed in split order in f64, then the epilogue
+hipError_t launch_ex_reduce(const float* P, void* y, bool yf32, bool gu, int M, int64_t nout, int64_t up_off,
+                            int64_t ld, int splits, hipStream_t s);
 // exact generic kernel, any M, scalar activation loads
 hipError_t launch_generic(const WeightView& w, const void* x, bool xf32, void* y, bool yf32, bool gu, int M,
                           int64_t nout, int64_t up_off, hipStream_t s);
@@ -222,6 +225,21 @@ hipError_t launch_q8act_tiled(const TilePlan& p, const WeightView& w, const uint
 size_t q8act_emit_counters(int64_t M, int64_t K, int64_t nout);
 hipError_t launch_q8act_dot_emit(const WeightView& w, const void* planes, void* y, bool yf32, int M, int64_t nout,
                                  uint32_t* counters, void* out_planes, hipStream_t s);
+// THQ_MODE_Q8ACT on the int8 matrix cores for many rows (k_q8act_gemm.hip):
+// Q4_K / Q8_0, K % 256 == 0, over the planes of launch_q8act_prepare; ws holds
+// the split partials
+struct QgPlan {
+    int mh = 0;               // 32-row halves per group (0: unsupported)
+    int groups = 0, splits = 0, cps = 0;  // row groups, K splits, 256-wide chunks per split
+    size_t workspace_bytes = 0;
+};
+QgPlan plan_q8act_gemm(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus);
+hipError_t launch_q8act_gemm(const QgPlan& p, const WeightView& w, const int8_t* xq, const float* xd,
+                             const int16_t* xb, void* y, bool yf32, bool gu, int M, int64_t nout, int64_t up_off,
+                             float* ws, hipStream_t s);
+// the same over a whole plane set (q8act_workspace_bytes)
+hipError_t launch_q8act_dot_gemm(const QgPlan& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
+                                 int M, int64_t nout, int64_t up_off, float* ws, hipStream_t s);
 // GGML blocks of the dot type (qtype 8 -> Q8_0 blocks, 12 -> Q8_K blocks)
 hipError_t launch_quantize_act(int qtype, const void* x, bool xf32, int64_t M, int64_t K, void* blocks,
                                hipStream_t s);
