@@ -32,6 +32,11 @@ def _gpu():
     torch.cuda.synchronize()
 
 
+@pytest.fixture(autouse=True)
+def _route(monkeypatch):
+    monkeypatch.setenv("THQ_GEMM_EX", "1")  # small calls too
+
+
 def weight(fmt, n, k, ctx=None):
     if fmt == "affine":
         wq, sb = rand_qlin_fast(n, k, seed=n + k)
@@ -123,6 +128,13 @@ def test_capture_without_scratch_and_replay():
             g.replay()
             torch.cuda.synchronize()
             assert rel(out, ref) <= 2e-7
+
+
+def test_rule(monkeypatch):
+    monkeypatch.delenv("THQ_GEMM_EX")
+    w = weight("q4_k", 4096, 4096)
+    assert thq.call_scratch_bytes(w, 2, x_dtype=torch.float32) == 0  # the scalar kernel
+    assert thq.call_scratch_bytes(w, 3, x_dtype=torch.float32) > 0
 
 
 def test_two_streams():

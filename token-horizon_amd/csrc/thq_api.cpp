@@ -418,12 +418,17 @@ thq::QgPlan q8act_gemm_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m, 
 
 // f32 rows: k_gemm_ex (every format, K in whole chunks) in row chunks whose
 // scratch (activation planes, split partials) stays within EX_MAX_MB and the
-// caller's cap, wherever the scalar generic kernel ran before: from 2 rows (Q6_K
-// from 1).  Both sides at M = 5 / 300: k_gemm_ex.hip.  THQ_GEMM_EX=0 turns it off.
+// caller's cap, where the scalar generic kernel ran before and the call is
+// large enough for its three launches (scalar / it, us: 2 rows of 3072 x 1024
+// 10.9 / 16.0, 2 rows of 4096 x 4096 Q4_K 17.6 / 17.1, Q6_K 18.7 / 21.6; 5 rows
+// 40.8 / 17.8, 41.8 / 21.9).  THQ_GEMM_EX: 0 never, 1 wherever supported
+// (tests), unset: that rule.
 constexpr size_t EX_MAX_MB = 512;
 bool plan_ex(const Call& c, Route& r) {
-    if (!c.ex || c.am || !aligned16(c.x) || env_flag_off("THQ_GEMM_EX")) return false;
+    if (!c.ex || c.am || !aligned16(c.x)) return false;
     const thq_weight* w = c.w;
+    const char* e = getenv("THQ_GEMM_EX");
+    if (e && *e ? *e != '1' : (double)c.m * (double)w->N * (double)w->K < 4.5e7) return false;
     const int qt = view(w).qtype;
     const size_t cap = std::min(c.scratch_cap, EX_MAX_MB << 20);
     int64_t rows = c.m;
