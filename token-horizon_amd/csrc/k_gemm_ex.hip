@@ -592,23 +592,29 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
 // K / 256 f32 adds would round more than the splits themselves do), then the
 // epilogue; four outputs per thread where rows are multiples of 4.
 template <int V, bool GU, typename YT>
-__global__ __launch_bounds__(256) void k_ex_reduce(const float* __restrict__ P, YT* __restrict__ Y, int M,
+__global__ __launch_bounds__(64) void k_ex_reduce(const float* __restrict__ P, YT* __restrict__ Y, int M,
                                                    int64_t nout, int64_t up_off, int64_t ld, int S) {
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+    const int64_t i = ((int64_t)blockIdx.x * 64 + threadIdx.x) * V;
     if (i >= nout) return;
     const int64_t m = blockIdx.y, step = (int64_t)M * ld;
     typedef float vec_t __attribute__((ext_vector_type(V)));
     double a[V] = {}, u[V] = {};
     const float* p = P + m * ld + i;
-    for (int s = 0; s < S; ++s, p += step) {
-        vec_t v, w;
-        __builtin_memcpy(&v, p, sizeof(v));
-        if (GU) __builtin_memcpy(&w, p + up_off, sizeof(w));
+    for (int s0 = 0; s0 < S; s0 += 8) {
+        vec_t v[8], w[8];
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-            a[j] += (double)v[j];
-            if (GU) u[j] += (double)w[j];
+        for (int s = 0; s < 8; ++s) {  // eight loads in flight; past S the last again, not added
+            const float* q = p + (int64_t)(s0 + s < S ? s0 + s : S - 1) * step;
+            __builtin_memcpy(&v[s], q, sizeof(vec_t));
+            if (GU) __builtin_memcpy(&w[s], q + up_off, sizeof(vec_t));
         }
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                a[j] += s0 + s < S ? (double)v[s][j] : 0.0;
+                if (GU) u[j] += s0 + s < S ? (double)w[s][j] : 0.0;
+            }
     }
 #pragma unroll
     for (int j = 0; j < V; ++j)
@@ -618,14 +624,14 @@ __global__ __launch_bounds__(256) void k_ex_reduce(const float* __restrict__ P, 
 template <bool GU, typename YT>
 hipError_t ex_reduce(const float* P, YT* y, int M, int64_t nout, int64_t up_off, int64_t ld, int S, hipStream_t s) {
     const bool v4 = !((nout | up_off | ld) & 3);
-    const int64_t bx = (nout + (v4 ? 1024 : 256) - 1) / (v4 ? 1024 : 256);
+    const int64_t bx = (nout + (v4 ? 256 : 64) - 1) / (v4 ? 256 : 64);
     for (int m0 = 0; m0 < M; m0 += 65535) {  // grid.y limit: row chunks read and write at their own offset
         const dim3 grid((unsigned)bx, (unsigned)(M - m0 < 65535 ? M - m0 : 65535));
         if (v4)
-            hipLaunchKernelGGL((k_ex_reduce<4, GU, YT>), grid, dim3(256), 0, s, P + m0 * ld, y + m0 * nout, M, nout,
+            hipLaunchKernelGGL((k_ex_reduce<4, GU, YT>), grid, dim3(64), 0, s, P + m0 * ld, y + m0 * nout, M, nout,
                                up_off, ld, S);
         else
-            hipLaunchKernelGGL((k_ex_reduce<1, GU, YT>), grid, dim3(256), 0, s, P + m0 * ld, y + m0 * nout, M, nout,
+            hipLaunchKernelGGL((k_ex_reduce<1, GU, YT>), grid, dim3(64), 0, s, P + m0 * ld, y + m0 * nout, M, nout,
                                up_off, ld, S);
     }
     return hipGetLastError();
