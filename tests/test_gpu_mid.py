@@ -143,3 +143,17 @@ def test_mid_affine(n, k, m):
     assert rel_row_err(y, rounded_ref(xf, wf)) <= 1e-4
     exact = xf.astype(np.float64) @ wf.astype(np.float64).T
     assert rel_row_err(y, exact) <= 1e-2
+
+
+@pytest.mark.parametrize("n,k,m", [(768, 512, 257), (1000, 1024, 300), (512, 2048, 384)])
+def test_router_takes_one_round_plans_to_384_rows(n, k, m, monkeypatch):
+    """Past 256 rows the router takes this kernel where its plan is one round of blocks: the bits of THQ_GEMM_MID=1."""
+    monkeypatch.delenv("THQ_GEMM_MID", raising=False)
+    w = thq.QTensor.from_gguf_bytes(O.Q4_K, weight_bytes(O.Q4_K, n, k, seed=31), n, k)
+    x = torch.from_numpy(O.bf16_round(activations(m, k, seed=32))).cuda().to(torch.bfloat16)
+    y = thq.matmul(w, x, torch.float32)
+    monkeypatch.setenv("THQ_GEMM_MID", "1")
+    assert torch.equal(y, thq.matmul(w, x, torch.float32))
+    monkeypatch.setenv("THQ_GEMM_MID", "0")
+    z = thq.matmul(w, x, torch.float32)
+    assert rel_row_err(y.cpu().numpy(), z.cpu().numpy()) <= 1e-5  # the same bf16 weights, another f32 order

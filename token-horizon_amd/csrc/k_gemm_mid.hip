@@ -430,6 +430,7 @@ MidPlan plan_gemm_mid(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int c
             }
         }
     }
+    p.us = best;
     p.mh = bmh;
     p.nt = bnt;
     p.nw = bnw;

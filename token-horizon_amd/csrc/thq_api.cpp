@@ -645,9 +645,10 @@ Route plan_route(const Call& c) {
         // then-GEMM route (4096 x 12288 at M = 4096: 369 against 388 us;
         // 12288 x 4096 keeps that route: 180 against 219 us at M = 2048); on
         // weights of at least 12288 x 4096 elements also from 768 rows, and
-        // gate/up from 384 (12288 x 4096 / 4096 x 12288 at M = 768: 107.6 /
+        // gate/up from 257 rows (12288 x 4096 / 4096 x 12288 at M = 768: 107.6 /
         // 106.7 against 136.3 / 115.4 us; gate/up 2 x 12288 x 4096 at M = 384
-        // / 512: 128.4 / 130.4 against 146.5 / 151.3 us; at M = 512 the plain
+        // / 512: 128.4 / 130.4 against 146.5 / 151.3 us, at M = 333: 126.1 against
+        // 134.5, so gate/up from 257, where the tile GEMM starts a second row block; at M = 512 the plain
         // shapes keep the tile GEMM: 72.0 / 70.9 against 78.8 / 84.9).  Its
         // K splits meet in the last block of each tile, so only with arrival
         // counters.  THQ_GEMM_RQ: 0 never, 1 wherever supported (tests),
@@ -655,7 +656,7 @@ Route plan_route(const Call& c) {
         const char* rqe = getenv("THQ_GEMM_RQ");
         const int rq_mode = rqe && *rqe ? atoi(rqe) : -1;
         const bool rq_big = w->N * w->K >= (int64_t)12288 * 4096 && r.kind == Kind::GEMM &&
-                            (m >= 768 || (c.gu && m >= 384));
+                            (m >= 768 || (c.gu && m >= 257));
         const bool rq_default = rq_big || (m >= 1024 && (r.kind == Kind::GEMM ||
                                                          (r.kind == Kind::GEMM_DQ && dq_mode == -1 && w->N < w->K)));
         if (q4 && !r.exact && r.kind != Kind::GEMM_FQ && rq_mode != 0 && (rq_mode == 1 || rq_default) &&
@@ -681,14 +682,26 @@ Route plan_route(const Call& c) {
         // weights of at most 4096 rows, where the tile GEMM's few tiles leave
         // CUs idle (4096 x 4096 at M = 160 / 256 / 384: 23.6 / 26.1 / 31.9
         // against 27.5 / 31.0 / 34.6 us; at 512: 36.9 against 35.6).
+        // At 257..384 rows, where the tile GEMM pays for 512, also wherever its
+        // plan is one round of blocks, or its estimate is under 1.2e-6 us per
+        // weight (the tile GEMM's and k_gemm_rq's least is 1.3e-6): 12288 x 4096
+        // at M = 257..320 54.4 against 70.5..73.4 us, 6144 x 4096 at M = 300 / 384
+        // 36.4 / 41.5 against 45.5 / 46.0, 4096 x 12288 60.8 / 62.0 against 66.0 /
+        // 67.9, gate/up 20480 x 2560 60.2 / 60.7 against 92.6 / 88.5, gate/up
+        // 24576 x 4096 at M = 300 112.9 against 126.6 (at 333: 158.9, not taken).
         // THQ_GEMM_MID: 0 never, 1 wherever supported (tests), unset: that rule
         const char* mde = getenv("THQ_GEMM_MID");
         const int mid_mode = mde && *mde ? atoi(mde) : -1;
         const int mid_max = w->N >= w->K ? (w->N == w->K && w->N <= 4096 ? 384 : 128) : 64;
         const bool mid_default = m >= 17 && m <= mid_max && r.kind == Kind::GEMM;
-        if (q4 && !r.exact && mid_mode != 0 && (mid_mode == 1 || mid_default)) {
+        const bool mid_maybe = m > 256 && m <= 384 && rq_mode != 1 &&
+                               (r.kind == Kind::GEMM || r.kind == Kind::GEMM_RQ);
+        if (q4 && !r.exact && mid_mode != 0 && (mid_mode == 1 || mid_default || mid_maybe)) {
             const thq::MidPlan mp = thq::plan_gemm_mid(v.qtype, m, w->N, w->K, c.gu, c.ctx->cus);
-            if (mp.mh > 0 && mp.workspace_bytes <= c.scratch_cap) {
+            const int64_t per = 32 * mp.nw * mp.nt, blocks = (w->N + per - 1) / per * mp.groups * mp.splits;
+            const bool ok = mid_mode == 1 || mid_default || blocks <= c.ctx->cus ||
+                            mp.us <= 1.2e-6 * (double)w->N * (double)w->K;
+            if (mp.mh > 0 && ok && mp.workspace_bytes <= c.scratch_cap) {
                 r.kind = Kind::GEMM_MID;
                 r.mp = mp;
                 r.scratch = mp.workspace_bytes;

@@ -113,6 +113,7 @@ hipError_t launch_gemv_wide(const WidePlan& p, const WeightView& w, const void* 
 struct MidPlan {
     int mh = 0, nt = 1, nw = 4, groups = 0;  // 32-row halves per group (2 or 4; 0: unsupported), column tiles per wave, waves per block, groups
     int splits = 0, cps = 0;      // K splits, 256-wide chunks per split
+    double us = 0.0;              // the planner's estimate
     size_t workspace_bytes = 0;   // split partials (f32 [splits][M][N])
 };
 MidPlan plan_gemm_mid(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus);
