@@ -1312,8 +1312,11 @@ int run_q8act_dot(thq_ctx* ctx, const thq_weight* w, thq_dtype dot_type, const v
         const thq::QgPlan qg = q8act_gemm_plan(ctx, w, m, gu);
         void* part = nullptr;
         bool ok = qg.groups > 0;
+        // held over both launches: another thread's call on this stream uses
+        // the same buffer, and may not come between the GEMM and its reduce
+        std::unique_lock<std::mutex> lk(ctx->mu, std::defer_lock);
         if (ok && qg.splits > 1) {
-            std::lock_guard<std::mutex> lk(ctx->mu);
+            lk.lock();
             part = side_scratch(ctx, s, qg.workspace_bytes);
             ok = part != nullptr;
         }
