@@ -30,8 +30,11 @@
  *    shared workspace: they (and the split sums of thq_matmul_q8act from 9 rows)
  *    take scratch that the context keeps per stream
  *    (at most 8 streams, until thq_destroy), so they stay re-entrant on
- *    distinct streams; where that cannot be had (more streams, growth under
- *    capture) they run the slower scalar kernel, which needs none.
+ *    distinct streams; where that cannot be had (more streams) they run the
+ *    slower scalar kernel, which needs none.  Captured ones need no warm-up
+ *    for it: each captured graph gets scratch of its own (at most 4 GiB per
+ *    context in all, kept until thq_destroy), so graphs may be replayed on any
+ *    streams, beside each other and beside eager calls.
  *  - W is [N, K] row-major (row n = output feature n), exactly the GGUF
  *    tensor layout QTensor::data() returns.  y[m, n] = sum_k x[m, k] * W[n, k].
  */

@@ -7,8 +7,9 @@ kernel it replaces measures 1.18e-7 .. 1.37e-7 over K = 1024 .. 17408, this
 one 0.8e-7 .. 1.33e-7; the reference's own f32-rounded weights add about 4e-8.
 Covered: the stacked form's edge (16 / 17 rows), whole and partial row groups,
 ragged outputs, one chunk and several K splits, bf16 output, rows of very
-large, very small and non-finite values, growth under capture (the general
-kernel runs), replays of a captured call, and calls on two streams.
+large, very small and non-finite values, captured calls (the eager call's
+bits, warmed up or not), graphs beside each other and beside eager calls, and
+calls on two streams.
 """
 import numpy as np
 import pytest
@@ -106,28 +107,59 @@ def test_extreme_rows(fmt, m):
     assert torch.equal(z[keep], y[keep])
 
 
-def test_capture_without_scratch_and_replay():
-    """A stream whose scratch would have to grow under capture takes the general kernel; one that has it, its own."""
+def captured(w, x, out, s):
+    g = torch.cuda.CUDAGraph()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s), torch.cuda.graph(g, stream=s):
+        thq.matmul(w, x, out=out)
+    return g
+
+
+def test_capture_takes_the_eager_kernel():
+    """A captured call runs the eager call's kernels (its bits), warmed up on its stream, on another, or not at all."""
     ctx = thq.Context(0)
     w, x = weight("q4_k", 256, 1024, ctx), rows(5, 1024)
-    ref = x.double() @ w.dequantize().double().T
-    for warm in (False, True):
-        s = torch.cuda.Stream()
-        out = torch.empty((5, 256), device="cuda")
-        s.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(s):
-            if warm:
-                thq.matmul(w, x, out=out)
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, stream=s):
-                thq.matmul(w, x, out=out)
+    out = torch.empty((5, 256), device="cuda")
+    s = torch.cuda.Stream()
+    gs = [captured(w, x, out, s)]  # the context's first call
+    ref = thq.matmul(w, x, torch.float32)  # warm on the default stream
+    gs.append(captured(w, x, out, s))
+    with torch.cuda.stream(s):
+        s.wait_stream(torch.cuda.default_stream())
+        thq.matmul(w, x[:2], torch.float32)  # the stream's own scratch is then too small for x
+    gs.append(captured(w, x, out, s))
+    for g in gs:
         for _ in range(3):
             out.fill_(float("nan"))
             torch.randn(64, 64, device="cuda") @ torch.randn(64, 64, device="cuda")
             torch.cuda.synchronize()
             g.replay()
             torch.cuda.synchronize()
-            assert rel(out, ref) <= 2e-7
+            assert torch.equal(out, ref)
+
+
+def test_graphs_beside_each_other_and_eager_calls():
+    """Graphs captured on one stream, replayed on others beside eager calls on that stream: every call's own bits."""
+    w = weight("q4_k", 2048, 1024)
+    xs = [rows(40, 1024, seed=40 + i) for i in range(3)]
+    ref = [thq.matmul(w, x, torch.float32) for x in xs]
+    torch.cuda.synchronize()
+    cap, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
+    out = [torch.empty_like(ref[0]) for _ in range(2)]
+    graphs = [captured(w, x, y, cap) for x, y in zip(xs, out)]
+    torch.cuda.synchronize()
+    kept, eager = [[], []], []
+    for _ in range(30):
+        for i, s in enumerate(others):
+            with torch.cuda.stream(s):
+                graphs[i].replay()
+                kept[i].append(out[i].clone())
+        with torch.cuda.stream(cap):
+            eager.append(thq.matmul(w, xs[2], torch.float32))
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(y, ref[i]) for y in kept[i])
+    assert all(torch.equal(y, ref[2]) for y in eager)
 
 
 def test_rule(monkeypatch):

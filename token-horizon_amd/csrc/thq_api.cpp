@@ -40,6 +40,16 @@ struct thq_side {
 
 constexpr size_t SIDE_MAX = 8;
 
+// scratch of one captured graph's calls on one stream (graph_scratch)
+struct thq_graph_side {
+    unsigned long long id = 0;  // the capture's
+    hipStream_t s = nullptr;
+    void* p = nullptr;
+    size_t bytes = 0;
+};
+
+constexpr size_t GRAPH_SIDE_BYTES = (size_t)4 << 30;  // in all, per context
+
 struct thq_ctx {
     int device = 0;
     void* scratch = nullptr;  // this device's copy of `scratch` (thq_init)
@@ -61,6 +71,8 @@ struct thq_ctx {
     // scratch of the routes that replaced scratch-free ones (side_scratch)
     thq_side side[SIDE_MAX];
     size_t nside = 0;
+    std::vector<thq_graph_side> graph_side;
+    size_t graph_side_bytes = 0;
 };
 
 struct thq_weight {
@@ -219,13 +231,59 @@ uint32_t* tile_counters(thq_ctx* ctx, int64_t n) {
     return p;
 }
 
+// hipMalloc under another stream's (or the caller's own) capture
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool swapped;
+    RelaxedCapture() : swapped(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~RelaxedCapture() {
+        if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
+void* side_malloc(size_t bytes) {
+    RelaxedCapture relaxed;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+// Side scratch under capture: a graph may be replayed on any stream, beside
+// other graphs and eager calls, so it shares no buffer with them.  Calls
+// captured on one stream of one capture run in order and do share.  Kept
+// until thq_destroy (replays may come until then).
+void* graph_scratch(thq_ctx* ctx, hipStream_t s, unsigned long long id, size_t bytes) {
+    for (const thq_graph_side& e : ctx->graph_side)
+        if (e.id == id && e.s == s && e.bytes >= bytes) return e.p;
+    if (bytes > GRAPH_SIDE_BYTES - ctx->graph_side_bytes) return nullptr;
+    try {
+        ctx->graph_side.reserve(ctx->graph_side.size() + 1);
+    } catch (...) {
+        return nullptr;
+    }
+    void* p = side_malloc(bytes);
+    if (!p) return nullptr;
+    ctx->graph_side.push_back(thq_graph_side{id, s, p, bytes});
+    ctx->graph_side_bytes += bytes;
+    return p;
+}
+
 // Scratch for f32 calls, which use no shared workspace: one buffer per stream, so that such calls
 // on distinct streams stay independent of each other and of the shared
 // workspace (caller holds ctx->mu).  At most SIDE_MAX streams, each buffer
-// kept until thq_destroy and grown like the workspace; null when it cannot be
-// had (too many streams, growth under stream capture, out of memory): the
-// caller then takes a route without it.
+// kept until thq_destroy and grown like the workspace; a captured call takes
+// its graph's own instead.  Null when it cannot be had (too many streams, the
+// graphs' bound, out of memory): the caller then takes a route without it.
 void* side_scratch(thq_ctx* ctx, hipStream_t s, size_t bytes) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(s, &st, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (st == hipStreamCaptureStatusActive) return graph_scratch(ctx, s, id, bytes);
+    if (st != hipStreamCaptureStatusNone) return nullptr;
     thq_side* at = nullptr;
     thq_side* const end = ctx->side + ctx->nside;
     for (thq_side* e = ctx->side; e != end; ++e)
@@ -238,18 +296,10 @@ void* side_scratch(thq_ctx* ctx, hipStream_t s, size_t bytes) {
             return e->p;
         }
     if (!at && ctx->nside >= SIDE_MAX) return nullptr;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
     size_t want = bytes + (bytes >> 3);
     if (at && want < 2 * at->bytes) want = 2 * at->bytes;
-    void* p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    void* const p = side_malloc(want);
+    if (!p) return nullptr;
     if (at) {
         ctx->retired.push_back(at->p);
         at->p = p;
@@ -880,13 +930,15 @@ int thq_init(int device, thq_ctx** out) {
 
 void thq_destroy(thq_ctx* ctx) {
     if (!ctx) return;
-    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || ctx->nside || !ctx->retired.empty()) {
+    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || ctx->nside || !ctx->graph_side.empty() ||
+        !ctx->retired.empty()) {
         DeviceGuard g(ctx->device);
         (void)hipDeviceSynchronize();
         if (ctx->ws) (void)hipFree(ctx->ws);
         if (ctx->emit_cnt) (void)hipFree(ctx->emit_cnt);
         if (ctx->tile_cnt) (void)hipFree(ctx->tile_cnt);
         for (size_t i = 0; i < ctx->nside; ++i) (void)hipFree(ctx->side[i].p);
+        for (const thq_graph_side& e : ctx->graph_side) (void)hipFree(e.p);
         for (void* p : ctx->retired) (void)hipFree(p);
     }
     delete ctx;
