@@ -28,13 +28,14 @@
  *    A call that grows the workspace cannot run under stream capture: warm
  *    every captured shape once beforehand.  Calls on f32 rows do not use the
  *    shared workspace: they (and the split sums of thq_matmul_q8act from 9 rows)
- *    take scratch that the context keeps per stream
- *    (at most 8 streams, until thq_destroy), so they stay re-entrant on
- *    distinct streams; where that cannot be had (more streams) they run the
- *    slower scalar kernel, which needs none.  Captured ones need no warm-up
- *    for it: each captured graph gets scratch of its own (at most 4 GiB per
- *    context in all, kept until thq_destroy), so graphs may be replayed on any
- *    streams, beside each other and beside eager calls.
+ *    take scratch of their own from the context, so they stay re-entrant on
+ *    distinct streams: a buffer per stream, grown like the workspace; past 16
+ *    streams a stream takes over another's and waits for its work.  Captured
+ *    ones need no warm-up for it: each captured graph gets scratch of its own
+ *    (at most 4 GiB per context in all, kept until thq_destroy), so graphs may
+ *    be replayed on any streams, beside each other and beside eager calls.
+ *    Where none can be had (out of memory, the graphs' bound, eager calls on
+ *    hipStreamPerThread) they run slower kernels that need none.
  *  - W is [N, K] row-major (row n = output feature n), exactly the GGUF
  *    tensor layout QTensor::data() returns.  y[m, n] = sum_k x[m, k] * W[n, k].
  */
@@ -305,11 +306,13 @@ size_t thq_noalloc_scratch_bytes(void);
  * (gate_up = 1) call of M rows would take, on the host, and returns the
  * context workspace bytes it needs (0 for routes with no scratch); no device
  * work.  thq_reserve grows the context workspace to at least
- * workspace_bytes, sets aside as much for the next stream that makes f32
- * calls (a capture stream, which cannot allocate), and the context's zeroed split-K arrival counters to at
+ * workspace_bytes and the context's zeroed split-K arrival counters to at
  * least `counters` entries (one per 32-row output tile of the widest
- * weight, and 32 per row of a top-k call, at most 65536), synchronously (hipMalloc, hipMemset, device synchronize); calls
- * whose needs fit then allocate nothing.  thq_workspace_bytes returns the
+ * weight, and 32 per row of a top-k call, at most 65536), synchronously
+ * (hipMalloc, hipMemset, device synchronize); calls on the workspace whose
+ * needs fit then allocate nothing.  Scratch that is not the workspace's (f32
+ * rows: the bytes reported are those of the stream's or graph's own) is
+ * allocated by the first call that needs it.  thq_workspace_bytes returns the
  * current workspace size. */
 int thq_call_scratch_bytes(thq_ctx* ctx, const thq_weight* w, int64_t m, thq_act x_type, uint32_t flags,
                            int gate_up, size_t* bytes);

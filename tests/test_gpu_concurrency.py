@@ -6,6 +6,7 @@ that share the workspace must be ordered on one stream and are not mixed
 here.  Calls from several threads on one stream are ordered there whatever
 scratch they use.  Streams keep the default priority.
 """
+import ctypes as C
 import threading
 
 import pytest
@@ -111,5 +112,52 @@ def test_two_threads_one_stream_prepared_q8act():
 
     run_threads([lambda: worker(0), lambda: worker(1)])
     torch.cuda.synchronize()
+    for ys, r in zip(out, ref):
+        assert all(torch.equal(y, r) for y in ys)
+
+
+def f32_case(n=2048, k=1024, m=40):
+    """A weight, and x / its product by the f16 matrix-core kernel (whose scratch the tests below are about)."""
+    ctx = thq.Context(0)
+    w = thq.QTensor.from_gguf_bytes(thq.Q4_K, weight_bytes(O.Q4_K, n, k, seed=76), n, k, ctx=ctx)
+    xs = [torch.from_numpy(activations(m, k, seed=80 + i)).cuda() for i in range(2)]
+    ref = [thq.matmul(w, x, torch.float32) for x in xs]
+    torch.cuda.synchronize()
+    return w, xs, ref
+
+
+def test_more_streams_than_scratch_buffers():
+    """f32 calls on 20 streams: the context keeps 16 buffers, the others wait for one; every call's own bits."""
+    w, xs, ref = f32_case()
+    streams = [torch.cuda.ExternalStream(s.cuda_stream) for s in (torch.cuda.Stream() for _ in range(20))]
+    assert len({s.cuda_stream for s in streams}) == 20
+    out = []
+    for rep in range(4):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                out.append((i & 1, thq.matmul(w, xs[i & 1], torch.float32)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, ref[i]) for i, y in out)
+
+
+def test_per_thread_stream(monkeypatch):
+    """hipStreamPerThread is one handle for a stream of each thread's own: its f32 calls take the kernel without
+    scratch."""
+    w, xs, _ = f32_case()
+    monkeypatch.setenv("THQ_GEMM_EX", "0")
+    ref = [thq.matmul(w, x, torch.float32) for x in xs]
+    monkeypatch.delenv("THQ_GEMM_EX")
+    out = [[torch.empty_like(ref[0]) for _ in range(100)] for _ in range(2)]
+    torch.cuda.synchronize()
+    per_thread, hip = C.c_void_p(2), C.CDLL("libamdhip64.so.7")  # the runtime that is loaded already
+
+    def worker(i):
+        for y in out[i]:
+            rc = thq.lib.thq_matmul(w.ctx.h, w.h, C.c_void_p(xs[i].data_ptr()), thq.ACT_F32, xs[i].shape[0],
+                                    C.c_void_p(y.data_ptr()), thq.ACT_F32, 0, per_thread)
+            assert rc == thq.OK, thq.last_error()
+        assert hip.hipStreamSynchronize(per_thread) == 0
+
+    run_threads([lambda: worker(0), lambda: worker(1)])
     for ys, r in zip(out, ref):
         assert all(torch.equal(y, r) for y in ys)

@@ -113,3 +113,16 @@ def test_ticket_matches_separate_reduce(monkeypatch, gu):
     torch.cuda.synchronize()
     for t in a:
         assert torch.equal(t, c)
+
+
+def test_reserve_allocates_the_workspace_alone():
+    """A reserve takes the bytes asked for (and the growth's eighth), once."""
+    ctx = thq.Context(0)
+    ctx.reserve(1 << 20)
+    size = 512 << 20
+    free = [torch.cuda.mem_get_info()[0]]
+    for _ in range(3):
+        ctx.reserve(size)
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] - free[1] <= size + size // 4
+    assert free[1] == free[2] == free[3]

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -30,15 +31,17 @@
 constexpr size_t THQ_NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[THQ_NOALLOC_SCRATCH_BYTES];
 
-// one stream's own scratch (open: made by thq_reserve, taken by the first stream that asks)
+// a side scratch buffer of eager calls on stream `s` (SideScratch)
 struct thq_side {
     hipStream_t s = nullptr;
-    bool open = false;
     void* p = nullptr;
     size_t bytes = 0;
+    hipEvent_t done = nullptr;  // the end of the last user's work, where `marked`
+    bool marked = false;
+    uint64_t used = 0;  // a count of uses, for the least recent one
 };
 
-constexpr size_t SIDE_MAX = 8;
+constexpr size_t SIDE_MAX = 16;
 
 // scratch of one captured graph's calls on one stream (graph_scratch)
 struct thq_graph_side {
@@ -68,9 +71,11 @@ struct thq_ctx {
     // zero between launches; grown like the workspace
     uint32_t* tile_cnt = nullptr;
     size_t tile_cnt_n = 0;
-    // scratch of the routes that replaced scratch-free ones (side_scratch)
+    // scratch of the routes that replaced scratch-free ones (SideScratch)
     thq_side side[SIDE_MAX];
     size_t nside = 0;
+    uint64_t side_uses = 0;
+    bool side_shared = false;  // more streams than buffers: every use is marked
     std::vector<thq_graph_side> graph_side;
     size_t graph_side_bytes = 0;
 };
@@ -269,46 +274,101 @@ void* graph_scratch(thq_ctx* ctx, hipStream_t s, unsigned long long id, size_t b
     return p;
 }
 
-// Scratch for f32 calls, which use no shared workspace: one buffer per stream, so that such calls
-// on distinct streams stay independent of each other and of the shared
-// workspace (caller holds ctx->mu).  At most SIDE_MAX streams, each buffer
-// kept until thq_destroy and grown like the workspace; a captured call takes
-// its graph's own instead.  Null when it cannot be had (too many streams, the
-// graphs' bound, out of memory): the caller then takes a route without it.
-void* side_scratch(thq_ctx* ctx, hipStream_t s, size_t bytes) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    unsigned long long id = 0;
-    if (hipStreamGetCaptureInfo(s, &st, &id) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (st == hipStreamCaptureStatusActive) return graph_scratch(ctx, s, id, bytes);
-    if (st != hipStreamCaptureStatusNone) return nullptr;
-    thq_side* at = nullptr;
-    thq_side* const end = ctx->side + ctx->nside;
-    for (thq_side* e = ctx->side; e != end; ++e)
-        if (!e->open && e->s == s) at = e;
-    if (at && at->bytes >= bytes) return at->p;
-    for (thq_side* e = ctx->side; !at && e != end; ++e)
-        if (e->open && e->bytes >= bytes) {
-            e->open = false;
-            e->s = s;
-            return e->p;
+// Scratch of a call that uses no shared workspace (f32 rows, the split sums of
+// prepared 8-bit dots), from construction to destruction, with ctx->mu held
+// over both and the call's launches between them.  An eager call takes its
+// stream's buffer, which the stream's order guards (a destroyed stream's
+// handle can come back, but hipStreamDestroy returns after the stream's work:
+// measured on both runtimes in use).  Past SIDE_MAX streams it takes the
+// buffer used least recently and waits for that one's last work; from then on
+// every use records an event (2.9 us of a small call, so not before).  Buffers
+// are kept until thq_destroy and grown like the workspace.  A captured call
+// takes its graph's own.  p is null when there is none to be had: out of
+// memory, past the graphs' bound, or on hipStreamPerThread, one handle for a
+// stream of each thread's, whose work neither an event nor a device
+// synchronize waited for once the thread was gone (measured).  The caller then
+// takes a route without scratch.
+struct SideScratch {
+    void* p = nullptr;
+
+    SideScratch(thq_ctx* ctx, hipStream_t stream, size_t bytes) : c(ctx), s(stream) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        unsigned long long id = 0;
+        if (hipStreamGetCaptureInfo(s, &st, &id) != hipSuccess) {
+            (void)hipGetLastError();
+            return;
         }
-    if (!at && ctx->nside >= SIDE_MAX) return nullptr;
-    size_t want = bytes + (bytes >> 3);
-    if (at && want < 2 * at->bytes) want = 2 * at->bytes;
-    void* const p = side_malloc(want);
-    if (!p) return nullptr;
-    if (at) {
-        ctx->retired.push_back(at->p);
-        at->p = p;
-        at->bytes = want;
-    } else {
-        ctx->side[ctx->nside++] = thq_side{s, false, p, want};
+        if (st == hipStreamCaptureStatusActive) p = graph_scratch(c, s, id, bytes);
+        if (st != hipStreamCaptureStatusNone || s == hipStreamPerThread) return;
+        thq_side *q = nullptr, *oldest = c->side;
+        for (thq_side* i = c->side; i != c->side + c->nside; ++i) {
+            if (i->s == s && (!q || i->used > q->used)) q = i;
+            if (i->used < oldest->used) oldest = i;
+        }
+        if (!q && c->nside < SIDE_MAX) {
+            q = &c->side[c->nside];
+            if (!q->done && hipEventCreateWithFlags(&q->done, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                q->done = nullptr;
+                return;
+            }
+            if (!(q->p = side_malloc(bytes + (bytes >> 3)))) return;
+            q->bytes = bytes + (bytes >> 3);
+            ++c->nside;
+        } else {
+            if (!q && !c->side_shared && !share()) return;
+            if (!q) q = oldest;
+            if (q->bytes < bytes && !grow(q, bytes)) return;
+            if (q->marked && hipStreamWaitEvent(s, q->done, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                return;
+            }
+        }
+        q->s = s;
+        q->used = ++c->side_uses;
+        e = q;
+        p = q->p;
     }
-    return p;
-}
+    ~SideScratch() {
+        if (!e) return;
+        e->marked = c->side_shared;
+        if (!e->marked || hipEventRecord(e->done, s) == hipSuccess) return;
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(s);  // the work's end is not marked: nobody may have the buffer before it
+    }
+    SideScratch(const SideScratch&) = delete;
+    SideScratch& operator=(const SideScratch&) = delete;
+
+private:
+    thq_ctx* c;
+    hipStream_t s;
+    thq_side* e = nullptr;
+
+    // the first stream past SIDE_MAX: no earlier use is marked, so wait for all of them
+    bool share() {
+        RelaxedCapture relaxed;
+        if (hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        c->side_shared = true;
+        return true;
+    }
+    bool grow(thq_side* q, size_t bytes) {
+        const size_t want = std::max(bytes + (bytes >> 3), 2 * q->bytes);  // retired bytes stay below the live size
+        try {
+            c->retired.reserve(c->retired.size() + 1);
+        } catch (...) {
+            return false;
+        }
+        void* const n = side_malloc(want);
+        if (!n) return false;
+        c->retired.push_back(q->p);
+        q->p = n;
+        q->bytes = want;
+        return true;
+    }
+};
 
 struct DeviceGuard {
     int prev = -1;
@@ -877,8 +937,8 @@ int run_matmul(const Call& c) {
     if (r.kind == Kind::NONE) return THQ_OK;
     std::lock_guard<std::mutex> lk(c.ctx->mu);
     if (r.kind == Kind::GEMM_EX) {
-        void* p = side_scratch(c.ctx, c.s, r.scratch);
-        if (p) return exec_route(c, r, p);
+        const SideScratch side(c.ctx, c.s, r.scratch);
+        if (side.p) return exec_route(c, r, side.p);
         Call d = c;
         d.ex = false;
         r = plan_route(d);
@@ -930,7 +990,7 @@ int thq_init(int device, thq_ctx** out) {
 
 void thq_destroy(thq_ctx* ctx) {
     if (!ctx) return;
-    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || ctx->nside || !ctx->graph_side.empty() ||
+    if (ctx->ws || ctx->emit_cnt || ctx->tile_cnt || ctx->side[0].done || !ctx->graph_side.empty() ||
         !ctx->retired.empty()) {
         DeviceGuard g(ctx->device);
         (void)hipDeviceSynchronize();
@@ -938,6 +998,8 @@ void thq_destroy(thq_ctx* ctx) {
         if (ctx->emit_cnt) (void)hipFree(ctx->emit_cnt);
         if (ctx->tile_cnt) (void)hipFree(ctx->tile_cnt);
         for (size_t i = 0; i < ctx->nside; ++i) (void)hipFree(ctx->side[i].p);
+        for (thq_side& q : ctx->side)
+            if (q.done) (void)hipEventDestroy(q.done);
         for (const thq_graph_side& e : ctx->graph_side) (void)hipFree(e.p);
         for (void* p : ctx->retired) (void)hipFree(p);
     }
@@ -1362,19 +1424,18 @@ int run_q8act_dot(thq_ctx* ctx, const thq_weight* w, thq_dtype dot_type, const v
     } else {
         const hipStream_t s = static_cast<hipStream_t>(stream);
         const thq::QgPlan qg = q8act_gemm_plan(ctx, w, m, gu);
-        void* part = nullptr;
-        bool ok = qg.groups > 0;
+        const bool split = qg.groups > 0 && qg.splits > 1;
         // held over both launches: another thread's call on this stream uses
         // the same buffer, and may not come between the GEMM and its reduce
         std::unique_lock<std::mutex> lk(ctx->mu, std::defer_lock);
-        if (ok && qg.splits > 1) {
+        std::optional<SideScratch> side;
+        if (split) {
             lk.lock();
-            part = side_scratch(ctx, s, qg.workspace_bytes);
-            ok = part != nullptr;
+            side.emplace(ctx, s, qg.workspace_bytes);
         }
-        if (ok)
+        if (qg.groups > 0 && (!split || side->p))
             e = thq::launch_q8act_dot_gemm(qg, view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0,
-                                           static_cast<float*>(part), s);
+                                           static_cast<float*>(split ? side->p : nullptr), s);
         else
             e = thq::launch_q8act_dot(view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0, s);
     }
@@ -1425,11 +1486,13 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
         return THQ_OK;
     }
     const thq::QgPlan qg = q8act_gemm_plan(ctx, fused, m, true);
-    void* part = qg.groups > 0 && qg.splits > 1 ? side_scratch(ctx, s, qg.workspace_bytes) : nullptr;
-    if (qg.groups > 0 && (qg.splits == 1 || part)) {
+    const bool split = qg.groups > 0 && qg.splits > 1;
+    std::optional<SideScratch> side;
+    if (split) side.emplace(ctx, s, qg.workspace_bytes);
+    if (qg.groups > 0 && (!split || side->p)) {
         // many rows: the same two launches on the int8 matrix cores
         hipError_t e = thq::launch_q8act_dot_gemm(qg, view(fused), buf_dev, y_dev, y_type == THQ_ACT_F32, true, (int)m,
-                                                  nout, nout, static_cast<float*>(part), s);
+                                                  nout, nout, static_cast<float*>(split ? side->p : nullptr), s);
         if (e == hipSuccess)
             e = thq::launch_q8act_prepare(12, y_dev, y_type == THQ_ACT_F32, m, nout, next_buf_dev, s);
         if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
@@ -1508,19 +1571,6 @@ int thq_reserve(thq_ctx* ctx, size_t workspace_bytes, int64_t counters) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     int rc = ensure_ws(ctx, workspace_bytes);
     if (rc) return rc;
-    if (workspace_bytes) {
-        // the same for the calls with a scratch of their own: a buffer that the
-        // next stream without one takes (a capture stream, which cannot allocate)
-        bool have = false;
-        for (size_t i = 0; i < ctx->nside; ++i) have |= ctx->side[i].open && ctx->side[i].bytes >= workspace_bytes;
-        if (!have && ctx->nside < SIDE_MAX) {
-            void* p = nullptr;
-            hipError_t e = hipMalloc(&p, workspace_bytes);
-            if (e != hipSuccess)
-                return fail(THQ_ENOMEM, "workspace hipMalloc(%zu): %s", workspace_bytes, hipGetErrorString(e));
-            ctx->side[ctx->nside++] = thq_side{nullptr, true, p, workspace_bytes};
-        }
-    }
     if (counters > 0 && !tile_counters(ctx, counters))
         return fail(THQ_ENOMEM, "arrival counters (%lld entries) could not be allocated", (long long)counters);
     HIP_TRY(hipDeviceSynchronize());
