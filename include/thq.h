@@ -32,7 +32,8 @@
  *    distinct streams: a buffer per stream, grown like the workspace; past 16
  *    streams a stream takes over another's and waits for its work.  Captured
  *    ones need no warm-up for it: each captured graph gets scratch of its own
- *    (at most 4 GiB per context in all, kept until thq_destroy), so graphs may
+ *    (at most THQ_GRAPH_SCRATCH_MB, 4096, per context in all, kept until
+ *    thq_destroy), so graphs may
  *    be replayed on any streams, beside each other and beside eager calls.
  *    Where none can be had (out of memory, the graphs' bound, eager calls on
  *    hipStreamPerThread) they run slower kernels that need none.

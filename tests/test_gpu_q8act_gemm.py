@@ -105,3 +105,38 @@ def test_rule_and_capture():
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, ref)
+
+
+def capture(f):
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s), torch.cuda.graph(g, stream=s):
+        return g, f()
+
+
+def test_captured_without_scratch(monkeypatch):
+    """Captures that get no graph scratch run the row-tile kernels, the emitting gate/up too, though no eager call of
+    this size has made its counters."""
+    ctx, ctx_ref = thq.Context(0), thq.Context(0)
+    h, k, m = 4096, 4096, 16
+    w = thq.QTensor.from_gguf_bytes(O.Q4_K, weight_bytes(O.Q4_K, 2 * h, k, seed=12), 2 * h, k, ctx=ctx)
+    x = torch.from_numpy(activations(m, k, seed=13)).cuda()
+    planes = thq.Q8Act(x, thq.Q8_K, ctx=ctx)
+    assert thq.call_scratch_bytes(w, m, torch.float32, thq.MODE_Q8ACT, True) > 8 * m * h  # split sums
+    planes.gate_up_silu_emit(w, torch.float32)  # warm
+    with monkeypatch.context() as mp:
+        mp.setenv("THQ_Q8ACT_GEMM", "0")
+        ref, nref = thq.Q8Act(x, thq.Q8_K, ctx=ctx_ref).gate_up_silu_emit(w, torch.float32)
+        pref = planes.matmul(w, torch.float32)
+    monkeypatch.setenv("THQ_GRAPH_SCRATCH_MB", "0")
+    g, (y, nxt, p) = capture(lambda: (*planes.gate_up_silu_emit(w, torch.float32), planes.matmul(w, torch.float32)))
+    for _ in range(3):
+        y.fill_(float("nan"))
+        p.fill_(float("nan"))
+        nxt.buf.zero_()
+        torch.randn(64, 64, device="cuda") @ torch.randn(64, 64, device="cuda")
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref) and torch.equal(p, pref)
+        assert torch.equal(nxt.buf, nref.buf)

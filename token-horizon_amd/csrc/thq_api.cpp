@@ -51,7 +51,7 @@ struct thq_graph_side {
     size_t bytes = 0;
 };
 
-constexpr size_t GRAPH_SIDE_BYTES = (size_t)4 << 30;  // in all, per context
+constexpr long GRAPH_SIDE_MB = 4096;  // in all, per context (THQ_GRAPH_SCRATCH_MB)
 
 struct thq_ctx {
     int device = 0;
@@ -261,7 +261,9 @@ void* side_malloc(size_t bytes) {
 void* graph_scratch(thq_ctx* ctx, hipStream_t s, unsigned long long id, size_t bytes) {
     for (const thq_graph_side& e : ctx->graph_side)
         if (e.id == id && e.s == s && e.bytes >= bytes) return e.p;
-    if (bytes > GRAPH_SIDE_BYTES - ctx->graph_side_bytes) return nullptr;
+    const char* mb = getenv("THQ_GRAPH_SCRATCH_MB");
+    const size_t most = (size_t)(mb && *mb ? std::max(0l, atol(mb)) : GRAPH_SIDE_MB) << 20;
+    if (bytes > most || ctx->graph_side_bytes > most - bytes) return nullptr;
     try {
         ctx->graph_side.reserve(ctx->graph_side.size() + 1);
     } catch (...) {
@@ -1486,15 +1488,19 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
         return THQ_OK;
     }
     const thq::QgPlan qg = q8act_gemm_plan(ctx, fused, m, true);
-    const bool split = qg.groups > 0 && qg.splits > 1;
-    std::optional<SideScratch> side;
-    if (split) side.emplace(ctx, s, qg.workspace_bytes);
-    if (qg.groups > 0 && (!split || side->p)) {
-        // many rows: the same two launches on the int8 matrix cores
-        hipError_t e = thq::launch_q8act_dot_gemm(qg, view(fused), buf_dev, y_dev, y_type == THQ_ACT_F32, true, (int)m,
-                                                  nout, nout, static_cast<float*>(split ? side->p : nullptr), s);
-        if (e == hipSuccess)
-            e = thq::launch_q8act_prepare(12, y_dev, y_type == THQ_ACT_F32, m, nout, next_buf_dev, s);
+    if (qg.groups > 0) {
+        // many rows: two launches as above, on the int8 matrix cores, or where
+        // their split sums find no scratch the row-tile kernels; neither needs
+        // the counters, whose growth a capture would not allow
+        const bool split = qg.splits > 1;
+        std::optional<SideScratch> side;
+        if (split) side.emplace(ctx, s, qg.workspace_bytes);
+        const bool yf32 = y_type == THQ_ACT_F32;
+        hipError_t e = split && !side->p
+                           ? thq::launch_q8act_dot(view(fused), buf_dev, y_dev, yf32, true, (int)m, nout, nout, s)
+                           : thq::launch_q8act_dot_gemm(qg, view(fused), buf_dev, y_dev, yf32, true, (int)m, nout, nout,
+                                                        static_cast<float*>(split ? side->p : nullptr), s);
+        if (e == hipSuccess) e = thq::launch_q8act_prepare(12, y_dev, yf32, m, nout, next_buf_dev, s);
         if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
         return THQ_OK;
     }
