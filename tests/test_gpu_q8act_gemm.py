@@ -140,3 +140,17 @@ def test_captured_without_scratch(monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(y, ref) and torch.equal(p, pref)
         assert torch.equal(nxt.buf, nref.buf)
+
+
+def test_many_rows_in_chunks():
+    """Split sums past 512 MiB: row chunks, each row's bits as in a call of its own chunk, prepared or not."""
+    n, k, m = 65536, 4352, 1100
+    w = thq.QTensor.from_gguf_bytes(O.Q4_K, np.tile(weight_bytes(O.Q4_K, 1024, k, seed=15).reshape(1024, -1), (64, 1)),
+                                    n, k)
+    x = torch.from_numpy(activations(m, k, seed=16)).cuda()
+    size = thq.call_scratch_bytes(w, m, torch.float32, thq.MODE_Q8ACT)
+    assert (256 << 20) < size <= (512 << 20) + 2 * m * k
+    y = thq.matmul(w, x, torch.float32, thq.MODE_Q8ACT)
+    parts = [thq.matmul(w, x[a:b], torch.float32, thq.MODE_Q8ACT) for a, b in ((0, 512), (512, 1024), (1024, m))]
+    assert torch.equal(y, torch.cat(parts))
+    assert torch.equal(thq.Q8Act(x, thq.Q8_K).matmul(w, torch.float32), y)

@@ -784,10 +784,19 @@ hipError_t launch_q8act_dot_tile(const TilePlan& p, const WeightView& w, const u
     return launch_q8act_tile(p, w, tiles, a.xq, a.xd, a.xb, y, yf32, gu, M, ws, cnt, s);
 }
 
-hipError_t launch_q8act_dot_gemm(const QgPlan& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
+hipError_t launch_q8act_dot_gemm(const QgRows& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
                                  int M, int64_t nout, int64_t up_off, float* ws, hipStream_t s) {
+    if (p.rows < 1) return hipErrorInvalidValue;
     const ActPlanes a = act_planes(w.qtype, const_cast<void*>(planes), M, w.K);
-    return launch_q8act_gemm(p, w, a.xq, a.xd, a.xb, y, yf32, gu, M, nout, up_off, ws, s);
+    const size_t yrow = (size_t)nout * (yf32 ? 4 : 2);
+    hipError_t e = hipSuccess;
+    for (int64_t r0 = 0; r0 < M && e == hipSuccess; r0 += p.rows) {
+        const int mm = (int)(M - r0 < p.rows ? M - r0 : p.rows);
+        const ActPlanes r = act_rows(a, w.qtype, w.K, r0);
+        e = launch_q8act_gemm(mm == p.rows ? p.p : p.last, w, r.xq, r.xd, r.xb, static_cast<char*>(y) + r0 * yrow, yf32,
+                              gu, mm, nout, up_off, ws, s);
+    }
+    return e;
 }
 
 hipError_t launch_q8act_tiled(const TilePlan& p, const WeightView& w, const uint8_t* tiles, const void* x, bool xf32,

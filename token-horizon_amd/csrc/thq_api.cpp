@@ -208,7 +208,10 @@ int ensure_ws(thq_ctx* ctx, size_t bytes) {
     if (want < 2 * ctx->ws_bytes) want = 2 * ctx->ws_bytes;  // retired bytes stay below the live size
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) return fail(THQ_ENOMEM, "workspace hipMalloc(%zu): %s", want, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's
+        return fail(THQ_ENOMEM, "workspace hipMalloc(%zu): %s", want, hipGetErrorString(e));
+    }
     if (ctx->ws) ctx->retired.push_back(ctx->ws);
     ctx->ws = p;
     ctx->ws_bytes = want;
@@ -433,6 +436,7 @@ struct Call {
     size_t scratch_cap = SIZE_MAX;  // routes needing more scratch are not planned
     bool counters = true;           // the caller can supply zeroed arrival counters
     bool ex = true;                 // k_gemm_ex may be planned (its scratch can be had)
+    bool qg = true;                 // k_q8act_gemm likewise
 };
 
 // an environment switch set to "0" (read on every call)
@@ -493,7 +497,7 @@ struct Route {
     thq::MidPlan mp;
     thq::ExPlan ep, ep_last;  // GEMM_EX: row chunks of ex_rows, and the last, partial one
     int ex_rows = 0;
-    thq::QgPlan qg;
+    thq::QgRows qg;
     bool exact = false;
     size_t scratch = 0;
 };
@@ -518,14 +522,28 @@ thq::TilePlan q8act_tile_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m
 // 16 / 24: 18.0 / 26.9 against 20.7 / 21.8; 4096 x 12288 at M = 9: 28.0 / 24.5;
 // 4096 x 4096 at M = 64 / 128: 16.9 / 29.4 against 19.9 / 25.0).
 // THQ_Q8ACT_GEMM: 0 never, 1 wherever supported (tests), unset: that rule.
-constexpr size_t QG_MAX_MB = 2048;  // of split partials
-thq::QgPlan q8act_gemm_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m, bool gu) {
+// Its split partials stay within `cap`: larger calls run in row chunks.
+constexpr size_t QG_MAX_BYTES = (size_t)512 << 20;
+thq::QgRows q8act_gemm_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m, bool gu, size_t cap = QG_MAX_BYTES) {
     const char* e = getenv("THQ_Q8ACT_GEMM");
     const double size = (double)m * (double)w->N * (double)w->K;
     const double least = w->qtype == THQ_Q8_0 ? (w->N < w->K ? 4.5e8 : 1.3e9) : (m >= 48 ? 1.5e8 : w->N < w->K ? 8e8 : 3e8);
-    if (e && *e ? *e != '1' : m < 9 || size < least) return thq::QgPlan{};
-    const thq::QgPlan p = thq::plan_q8act_gemm(view(w).qtype, m, w->N, w->K, gu, ctx->cus);
-    return p.workspace_bytes <= QG_MAX_MB << 20 ? p : thq::QgPlan{};
+    if (e && *e ? *e != '1' : m < 9 || size < least) return thq::QgRows{};
+    cap = std::min(cap, QG_MAX_BYTES);
+    auto plan = [&](int64_t rows) { return thq::plan_q8act_gemm(view(w).qtype, rows, w->N, w->K, gu, ctx->cus); };
+    thq::QgRows r;
+    int64_t rows = m;
+    r.p = plan(rows);
+    while ((r.p.groups == 0 || r.p.workspace_bytes > cap) && rows > 64) {
+        rows = std::max<int64_t>(64, rows / 2 / 64 * 64);
+        r.p = plan(rows);
+    }
+    r.last = m % rows ? plan(m % rows) : r.p;
+    if (r.p.groups == 0 || r.last.groups == 0) return thq::QgRows{};
+    r.workspace_bytes = std::max(r.p.workspace_bytes, r.last.workspace_bytes);
+    if (r.workspace_bytes > cap) return thq::QgRows{};
+    r.rows = (int)rows;
+    return r;
 }
 
 // f32 rows: k_gemm_ex (every format, K in whole chunks) in row chunks whose
@@ -584,12 +602,14 @@ Route plan_route(const Call& c) {
             r.scratch = align_up(r.scratch, 256) + tp.workspace_bytes;
             return r;
         }
-        const thq::QgPlan qg = q8act_gemm_plan(c.ctx, w, m, c.gu);
-        const size_t need = align_up(r.scratch, 256) + qg.workspace_bytes;
-        if (qg.groups > 0 && need <= c.scratch_cap) {
-            r.kind = Kind::Q8ACT_GEMM;
-            r.qg = qg;
-            r.scratch = need;
+        const size_t planes = align_up(r.scratch, 256);
+        if (c.qg && planes <= c.scratch_cap) {
+            const thq::QgRows qg = q8act_gemm_plan(c.ctx, w, m, c.gu, c.scratch_cap - planes);
+            if (qg.rows > 0) {
+                r.kind = Kind::Q8ACT_GEMM;
+                r.qg = qg;
+                r.scratch = planes + qg.workspace_bytes;
+            }
         }
         return r;
     }
@@ -947,6 +967,13 @@ int run_matmul(const Call& c) {
     }
     if (r.scratch) {
         rc = ensure_ws(c.ctx, r.scratch);
+        if (rc && r.kind == Kind::Q8ACT_GEMM) {
+            // no room for its split sums: the row-tile kernels need the planes alone
+            Call d = c;
+            d.qg = false;
+            r = plan_route(d);
+            rc = ensure_ws(c.ctx, r.scratch);
+        }
         if (rc) return rc;
     }
     uint32_t* cnt = nullptr;
@@ -1425,8 +1452,8 @@ int run_q8act_dot(thq_ctx* ctx, const thq_weight* w, thq_dtype dot_type, const v
                                        static_cast<float*>(ctx->ws), cnt, static_cast<hipStream_t>(stream));
     } else {
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        const thq::QgPlan qg = q8act_gemm_plan(ctx, w, m, gu);
-        const bool split = qg.groups > 0 && qg.splits > 1;
+        const thq::QgRows qg = q8act_gemm_plan(ctx, w, m, gu);
+        const bool split = qg.workspace_bytes > 0;
         // held over both launches: another thread's call on this stream uses
         // the same buffer, and may not come between the GEMM and its reduce
         std::unique_lock<std::mutex> lk(ctx->mu, std::defer_lock);
@@ -1435,7 +1462,7 @@ int run_q8act_dot(thq_ctx* ctx, const thq_weight* w, thq_dtype dot_type, const v
             lk.lock();
             side.emplace(ctx, s, qg.workspace_bytes);
         }
-        if (qg.groups > 0 && (!split || side->p))
+        if (qg.rows > 0 && (!split || side->p))
             e = thq::launch_q8act_dot_gemm(qg, view(w), buf, y, yt == THQ_ACT_F32, gu, (int)m, nout, gu ? nout : 0,
                                            static_cast<float*>(split ? side->p : nullptr), s);
         else
@@ -1487,12 +1514,12 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
         if (e != hipSuccess) return fail(THQ_EHIP, "kernel launch: %s", hipGetErrorString(e));
         return THQ_OK;
     }
-    const thq::QgPlan qg = q8act_gemm_plan(ctx, fused, m, true);
-    if (qg.groups > 0) {
+    const thq::QgRows qg = q8act_gemm_plan(ctx, fused, m, true);
+    if (qg.rows > 0) {
         // many rows: two launches as above, on the int8 matrix cores, or where
         // their split sums find no scratch the row-tile kernels; neither needs
         // the counters, whose growth a capture would not allow
-        const bool split = qg.splits > 1;
+        const bool split = qg.workspace_bytes > 0;
         std::optional<SideScratch> side;
         if (split) side.emplace(ctx, s, qg.workspace_bytes);
         const bool yf32 = y_type == THQ_ACT_F32;

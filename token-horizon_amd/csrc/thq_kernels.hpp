@@ -238,8 +238,15 @@ QgPlan plan_q8act_gemm(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int 
 hipError_t launch_q8act_gemm(const QgPlan& p, const WeightView& w, const int8_t* xq, const float* xd,
                              const int16_t* xb, void* y, bool yf32, bool gu, int M, int64_t nout, int64_t up_off,
                              float* ws, hipStream_t s);
+// row chunks of one call, each with its plan (the last may be partial); they
+// run in stream order, so they share the partials
+struct QgRows {
+    int rows = 0;  // per chunk (0: none planned)
+    QgPlan p, last;
+    size_t workspace_bytes = 0;
+};
 // the same over a whole plane set (q8act_workspace_bytes)
-hipError_t launch_q8act_dot_gemm(const QgPlan& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
+hipError_t launch_q8act_dot_gemm(const QgRows& p, const WeightView& w, const void* planes, void* y, bool yf32, bool gu,
                                  int M, int64_t nout, int64_t up_off, float* ws, hipStream_t s);
 // GGML blocks of the dot type (qtype 8 -> Q8_0 blocks, 12 -> Q8_K blocks)
 hipError_t launch_quantize_act(int qtype, const void* x, bool xf32, int64_t M, int64_t K, void* blocks,
