@@ -269,9 +269,11 @@ int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype
  *              runs a bf16 MFMA GEMM on it, the engine's "dequant + bf16
  *              matmul" prefill route
  *   Q6_K under THQ_MODE_EXACT_W past 64 rows runs the exact decode GEMV in
- *   groups of 16 rows.  x f32 with M >= 2 and K a multiple of 256 runs on
- *   the f16 matrix cores, each row as two f16 planes, weights exact, no less
- *   precise than f32 dots; the remaining shapes run an exact scalar f32 path.
+ *   groups of 16 rows.  x f32 with M >= 2 (Q6_K: M >= 1) and K a multiple
+ *   of 256 runs, where the call is large enough, on the f16 matrix cores, each
+ *   row as three f16 planes that hold every bit of it, weights exact (relative
+ *   error against 64-bit sums over N(0, 1) rows at most 1.0e-7, f32 dots
+ *   1.4e-7); the remaining shapes run an exact scalar f32 path.
  * THQ_MODE_Q8ACT instead reproduces candle's default CPU k_quants::matmul:
  * x rows are quantized as thq_quantize_act does (into the context
  * workspace), every block dot is exact in integers and scaled in f32; only

@@ -3,13 +3,14 @@ plain and gate/up, against the f64 product with the library's f32
 dequantization (pinned bit-exact elsewhere).
 
 Bound: relative error of the whole result (2-norm) <= 2e-7.  The scalar f32
-kernel it replaces measures 1.18e-7 .. 1.37e-7 over K = 1024 .. 17408, this
-one 0.8e-7 .. 1.33e-7; the reference's own f32-rounded weights add about 4e-8.
-Covered: the stacked form's edge (16 / 17 rows), whole and partial row groups,
-ragged outputs, one chunk and several K splits, bf16 output, rows of very
-large, very small and non-finite values, captured calls (the eager call's
-bits, warmed up or not), graphs beside each other and beside eager calls, and
-calls on two streams.
+kernel it replaces measures 1.18e-7 .. 1.37e-7 over N(0, 1) rows, K = 1024 ..
+17408, this one 0.67e-7 .. 1.0e-7; the reference's own f32-rounded weights add
+about 4e-8.  Covered: the edges of the stacked forms (8 / 9, 16 / 17 rows),
+whole and partial row groups, ragged outputs, one chunk and several K splits,
+bf16 output, rows of very large, very small and non-finite values, every bit
+of x, values beside outliers, captured calls (the eager call's bits, warmed up
+or not), graphs beside each other and beside eager calls, and calls on two
+streams.
 """
 import numpy as np
 import pytest
@@ -57,7 +58,7 @@ def rel(y, ref):
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-@pytest.mark.parametrize("m,n,k", [(2, 40, 256), (16, 300, 1792), (17, 512, 1024), (33, 257, 2048), (70, 1000, 4096),
+@pytest.mark.parametrize("m,n,k", [(2, 40, 256), (8, 96, 512), (9, 130, 768), (16, 300, 1792), (17, 512, 1024), (33, 257, 2048), (70, 1000, 4096),
                                    (3, 96, 17408)])
 def test_rows_match_f64(fmt, m, n, k):
     w, x = weight(fmt, n, k), rows(m, k)
@@ -91,7 +92,7 @@ def test_extreme_rows(fmt, m):
     x[0] *= 1e30
     x[1] *= 1e-33
     x[2] = 0.0
-    x[3, 5] = 3e4 * x[3].abs().max()  # one outlier: the rest still carries
+    x[3, 5] = 3e4 * x[3].abs().max()
     ref = x.double() @ w.dequantize().double().T
     y = thq.matmul(w, x, torch.float32)
     for i in (0, 1, 3, 4):
@@ -105,6 +106,54 @@ def test_extreme_rows(fmt, m):
     assert torch.equal(z[1][wd[:, 9] != 0], torch.sign(wd[:, 9][wd[:, 9] != 0]) * float("inf"))
     keep = [i for i in range(m) if i not in (1, 4)]
     assert torch.equal(z[keep], y[keep])
+
+
+def wide_rows(m, k, seed):
+    """Rows of every spread: N(0, 1), up to 1e+-5 and 1e+-35 in one row, and a few values of 1e-12 and 1e9 beside N(0, 1)."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn((m, k), generator=g)
+    ten = torch.rand((m, k), generator=g) * 2 - 1
+    x[1::4] *= 10 ** (5 * ten[1::4])
+    x[2::4] *= 10 ** (35 * ten[2::4])
+    few = torch.rand((m, k), generator=g)
+    x[3::4][few[3::4] < 4 / k] *= 1e9
+    x[3::4][few[3::4] > 1 - 8 / k] *= 1e-12
+    x[0, :7] = torch.tensor([0.0, -0.0, 1e-45, -1e-38, 3e38, 1.0, 2.0**-149])
+    return x.cuda()
+
+
+@pytest.mark.parametrize("m", [2, 5, 8, 12, 16, 40])
+def test_every_bit_of_x(m):
+    """An identity weight (Q8_0: d = 1, one code of 1 per row) returns x itself."""
+    n = k = 768
+    blk = np.zeros((n, k // 32, 34), np.uint8)
+    blk[:, :, :2] = np.array([1.0], np.float16).view(np.uint8)
+    blk[np.arange(n), np.arange(n) // 32, 2 + np.arange(n) % 32] = 1
+    w = thq.QTensor.from_gguf_bytes(O.Q8_0, blk.reshape(n, -1), n, k)
+    for seed in range(3):
+        x = wide_rows(m, k, seed)
+        assert torch.equal(thq.matmul(w, x, torch.float32), x)
+
+
+@pytest.mark.parametrize("m", [5, 12, 40])
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_values_beside_outliers(fmt, m, monkeypatch):
+    """Each output against the size of its own products, not the row's: what an outlier adds where its weight is
+    small is no more than a f32 dot's rounding of the products that are there.  The bound is four times the scalar
+    kernel's largest error (4.0e-7 .. 5.5e-7; this one measures 5.2e-7 .. 1.02e-6)."""
+    n, k = 768, 1024
+    w, x = weight(fmt, n, k), wide_rows(m, k, seed=50)
+    x[0, 4] = 1.0  # 3e38 would overflow the products
+    x[2::4] *= 1e-2
+    wd = w.dequantize().double()
+    ref = x.double() @ wd.T
+    size = (x.double().square() @ wd.square().T).sqrt()
+    err = {}
+    for v in ("0", "1"):
+        monkeypatch.setenv("THQ_GEMM_EX", v)
+        err[v] = float(((thq.matmul(w, x, torch.float32).double() - ref).abs() / size).max())
+    print(f"[outliers] {fmt} m={m}: scalar {err['0']:.3g} planes {err['1']:.3g}", flush=True)
+    assert err["1"] <= 4 * err["0"]
 
 
 def captured(w, x, out, s):
@@ -192,6 +241,8 @@ def test_many_rows_in_chunks():
     w, x = weight("affine", n, k), rows(m, k, seed=9)
     assert thq.call_scratch_bytes(w, m, x_dtype=torch.float32) <= 512 << 20
     y = thq.matmul(w, x, torch.float32)
+    parts = [thq.matmul(w, x[a:b], torch.float32) for a, b in ((0, 512), (512, 1024), (1024, m))]
+    assert torch.equal(y, torch.cat(parts))
     pick = np.r_[0, 511, 512, 1023, 1024, 1099]
     ref = x[pick].double() @ w.dequantize().double().T
     assert rel(y[pick], ref) <= 2e-7

@@ -1,44 +1,52 @@
 // k_gemm_ex.hip — f32 activations of any row count past 1 on the f16 matrix
-// cores, exact weights, no less precise than f32 dots.
+// cores, every bit of x and of the weights.
 //
 // Role: candle's f32 QMatMul::forward on GGUF models (engine/src/
 // model.rs:551-562) over prompts and verify steps.  Before it, every f32 call
 // with M > 1 ran k_gemv_generic: scalar f32 dots, the weight dequantized again
 // for every 8 rows (Q4_K gate/up + down of 4096 / 12288 at M = 300: 19.2 ms,
-// now 0.41 ms; a decoder layer at M = 5: 424 us, now 102 us).
+// now 0.47 ms; a decoder layer at M = 5: 424 us, now 105 us).
 //
 // Activations (k_xplanes, one launch per call): each row is scaled by a power
-// of two so that its largest magnitude lies in [2^14, 2^15), then written as
-// two f16 planes, x0 = f16(x) and x1 = f16(x - x0): x0 + x1 is x to 2^-24 of
-// it, or to 2^-40 of the row's largest value where x1 is subnormal (the
-// matrix cores do not flush it).  The weights' integers are exact in f16
-// (Q4_K: sc (q - 8), at most 504; affine: q - 8; Q8_0: q; Q6_K: code - 32),
-// so each product is exact in f32.
+// of two and written as three f16 planes, x0 = f16(x), x1 = f16(2^11 (x - x0)),
+// x2 = 2^11 (x - x0) - x1, which hold every f32 from the row's largest down to
+// 2^-26 of it exactly (the matrix cores do not flush subnormals).  Two planes
+// hold 23 bits: one in four f32 values loses its last, and a third of their
+// MFMAs is what the 24th costs (the MLP above 0.41 ms, the layer 102 us).
+// What the planes do not hold (smaller values, Inf, NaN, a few outliers that
+// would push the rest out of their range) is listed per row and dotted in f32
+// with the weight as the scalar kernel forms it.  The weights' integers are
+// exact in f16 (Q4_K: sc (q - 8), at most 504; affine: q - 8; Q8_0: q; Q6_K:
+// code - 32), so each product is exact in f32.  The offsets of the 4-bit
+// weights are f32 factors times f32 sums of x.
 //
 // Sums: a 64-wide part (Q8_0: each 32-wide block of it, Q6_K: each 16-wide
-// group) is summed by the matrix core from zero, each plane by itself: a
-// chain that starts from the small plane's sum loses its low bits to the
-// alignment with the large plane's products (Q6_K, K = 17408: 2.7e-7 in
-// place of 1.1e-7).  The parts are scaled and added in f32 over at most
-// EX_CPS chunks of 256, the K splits in f64.  Relative error against 64-bit
-// sums (N(0, 1) rows, 2048 outputs, K = 1024 .. 17408): 0.8e-7 .. 1.33e-7; the
-// scalar kernel's is 1.18e-7 .. 1.37e-7, which fixes EX_CPS.
+// group) is summed by the matrix core from zero, x0 by itself: a chain that
+// starts from the small planes' sum loses its low bits to the alignment with
+// the large plane's products (Q6_K, K = 17408: 2.7e-7 in place of 1.1e-7).  The
+// parts are scaled and added in f32 over at most EX_CPS chunks of 256, the K
+// splits in f64.  Relative error against 64-bit sums (2-norm, 2048 outputs, K =
+// 1024 .. 17408): N(0, 1) rows 0.67e-7 .. 1.0e-7, the scalar kernel 1.19e-7 ..
+// 1.36e-7; N(0, 1) times exp(N(0, 4)) 0.8e-7 .. 1.42e-7 against 0.95e-7 ..
+// 1.35e-7.  As for f32 dots the error is that of sums of the products' size,
+// here of x with the integers as centred above: a weight that is zero or small
+// because its offset cancels a code (4-bit formats) counts with the code.
 //
 // Block = 4 waves; a wave owns two 32-row column tiles of weight rows
 // (gate/up: the gate and the up rows of the same 32 outputs) and streams them
-// into registers half a chunk ahead, converting each 64-wide part once for
-// the group's rows.  The rows' planes go chunk by chunk into LDS by
-// direct-to-LDS copies, the next chunk's while the current one computes; one
-// A operand read feeds two MFMAs.  Groups of 32 rows; up to 16 rows (ST) the
-// two planes are stacked in one 32-row operand and added in the epilogue,
-// half the MFMAs.  Groups of 64 rows spill or leave one wave per SIMD (gate/up
-// of the MLP above: 335 .. 358 against 268 .. 296 us).  Bound: VALU (the
-// conversion, ~2 instructions per weight and 32 rows) at prompts, the weight
-// stream's latency at verify sizes.
+// into registers a chunk ahead, half a chunk at a time, converting each
+// 64-wide part once for the group's rows.  The rows' planes go half a chunk at
+// a time into LDS by direct-to-LDS copies, the next half's while the current
+// one computes.  Groups of R = 32 rows; up to 16 (8) rows the planes are
+// stacked in two (one) 32-row operands and added in the epilogue, two thirds
+// (one third) of the MFMAs.  No instance spills.  Bound at prompts: gate/up of
+// 24576 x 4096 at M = 300 (280 us) keeps the VALU busy 42 % and the matrix cores
+// 35 % of the time with two waves per SIMD, 33 % of a wave's time in waits; the
+// conversion repeats per 32 rows.  At verify sizes: latency (one to six chunks
+// a block, 20 % waits, 7 % MFMA).
 #include "thq_dev.hpp"
 #include "thq_kernels.hpp"
 
-#include <climits>
 #include <type_traits>
 
 namespace thq {
@@ -49,8 +57,16 @@ typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t ex_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t ex_u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int EX_NONFINITE = INT_MIN;  // a row's exponent slot: the row holds Inf or NaN
-constexpr int EX_CPS = 6;              // chunks per K split (the accumulators' error, above)
+constexpr float EX_UP = 2048.0f;  // planes 1 and 2 hold 2^11 of what they stand for
+constexpr int EX_CPS = 6;         // chunks per K split (the accumulators' error, above)
+constexpr int EX_LIST = 32;       // listed elements per row; more, and the whole row is dotted in f32
+constexpr int EX_OUT = 8;         // outliers per row that do not set its scale
+
+// an element that the planes do not hold
+struct ExItem {
+    int k;
+    float x;
+};
 
 // ------------------------------------------------------------------ activation planes
 __device__ __forceinline__ float dpp_quad(float v) {  // sum over each quad of lanes
@@ -61,95 +77,164 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
     const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
     v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
-// A block per row: the row's largest magnitude, then its planes P [2][M][K],
-// its exponent E [M], and the sums the offset of a 4-bit weight multiplies:
-// Q4_K: SS [M][K/256][2][8] f16, 2^-6 of the scaled row's 32-wide sums in two
-// pieces; affine: SA [K/64][mpad] f32 64-wide sums.  A row that holds Inf or
-// NaN gets zero planes and EX_NONFINITE (k_gemm_ex dots it in f32).
-// Bound: latency (the row is read once, kept in registers up to K = 16384).
-constexpr int XP_T = 512, XP_KEEP = 4;
-template <int QT>
+// A block per row: its exponent E [M] (the planes hold x 2^-E), its planes
+// P [3][M][K], its list (LC [M]: so many items of LK [M][EX_LIST] in ascending
+// order, or -1 for the whole row), and for 4-bit weights SA [K/SB][mpad], the
+// f32 sums of the scaled row's SB-wide pieces that a weight's offset
+// multiplies (Q4_K: SB = 32, affine: 64).  E puts the row's largest magnitude
+// into [2^14, 2^15), or the largest once up to EX_OUT outliers, each level
+// more than 64 times the rest, are left out.  Listed: outliers, Inf, NaN, and
+// what the planes would round.  Bound: latency (the row is read once, KEEP
+// 8-wide pieces a thread kept in registers; 512 threads to K = 4096, 1024 past
+// it: 5 rows of 12288 1 us less than with 512, 300 rows of 4096 3.5 us more).
+template <int QT, int XP_T, int XP_KEEP>
 __global__ __launch_bounds__(XP_T) void k_xplanes(const float* __restrict__ X, int K, int64_t plane, h8_t* __restrict__ P,
-                                                  int* __restrict__ E, _Float16* __restrict__ SS,
+                                                  int* __restrict__ E, int* __restrict__ LC, ExItem* __restrict__ LK,
                                                   float* __restrict__ SA, int64_t mpad) {
-    __shared__ float red[XP_T / 64];
+    __shared__ float tops[2][XP_T / 64];
+    __shared__ int counts[2][XP_T / 64];
+    __shared__ int nlist;
+    __shared__ ExItem list[EX_LIST];
     const int64_t row = blockIdx.x;
     const float* x = X + row * K;
     const int n8 = K >> 3, tid = threadIdx.x;
+    if (tid == 0) nlist = 0;  // read after the first scan's barrier
     float v[XP_KEEP][8];
-    float mx = 0.0f;
-    bool bad = false;
-    auto scan = [&](const float (&a)[8]) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float m = fabsf(a[i]);
-            bad |= !(m <= 3.402823466e+38f);
-            mx = fmaxf(mx, m);
-        }
-    };
 #pragma unroll
     for (int j = 0; j < XP_KEEP; ++j) {
         const int p = tid + j * XP_T;
-        if (p < n8) {
-            load8(x + 8 * p, v[j]);
-            scan(v[j]);
+        if (p < n8) load8(x + 8 * p, v[j]);
+    }
+    auto each = [&](auto&& f) {  // the thread's 8-wide pieces
+#pragma unroll
+        for (int j = 0; j < XP_KEEP; ++j) {
+            const int p = tid + j * XP_T;
+            if (p < n8) f(p, v[j]);
         }
-    }
-    for (int p = tid + XP_KEEP * XP_T; p < n8; p += XP_T) {
-        float a[8];
-        load8(x + 8 * p, a);
-        scan(a);
-    }
-    if (bad) mx = INFINITY;
+        for (int p = tid + XP_KEEP * XP_T; p < n8; p += XP_T) {
+            float a[8];
+            load8(x + 8 * p, a);
+            f(p, a);
+        }
+    };
+    // A scan: this wave's largest magnitude below cut, and how many of its
+    // values lie in [from, lim); then every wave's.  (Magnitudes compare as
+    // their bits.)
+    int turn = 0;
+    auto wave_top = [&](float cut) {
+        uint32_t m = 0;
+        each([&](int, const float (&a)[8]) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = red[0];
+            for (int i = 0; i < 8; ++i) m = max(m, fabsf(a[i]) < cut ? __float_as_uint(fabsf(a[i])) : 0u);  // not NaN
+        });
+        m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xF, 0xF, false));
+        m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x140, 0xF, 0xF, false));
+        uint32_t w = 0;
 #pragma unroll
-    for (int i = 1; i < XP_T / 64; ++i) mx = fmaxf(mx, red[i]);
-    const bool fin = mx < INFINITY;
-    const int e = fin && mx > 0.0f ? ilogbf(mx) - 14 : 0;
-    if (tid == 0) E[row] = fin ? e : EX_NONFINITE;
+        for (int i = 0; i < 4; ++i) w = max(w, (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * i));
+        return __uint_as_float(w);
+    };
+    auto wave_count = [&](float from, float lim) {
+        int c = 0;
+        each([&](int, const float (&a)[8]) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) c += fabsf(a[i]) >= from && fabsf(a[i]) < lim;
+        });
+        c += __builtin_amdgcn_mov_dpp(c, 0xB1, 0xF, 0xF, false);
+        c += __builtin_amdgcn_mov_dpp(c, 0x4E, 0xF, 0xF, false);
+        c += __builtin_amdgcn_mov_dpp(c, 0x141, 0xF, 0xF, false);
+        c += __builtin_amdgcn_mov_dpp(c, 0x140, 0xF, 0xF, false);
+        int w = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w += __builtin_amdgcn_readlane(c, 16 * i);
+        return w;
+    };
+    auto meet = [&](float m, int c) {
+        if ((tid & 63) == 0) {
+            tops[turn][tid >> 6] = m;
+            counts[turn][tid >> 6] = c;
+        }
+        __syncthreads();
+    };
+    float lim = INFINITY, top = 0.0f;  // the planes hold magnitudes below lim
+    int crowd = 0;                     // of the wave that holds the top: values within 64 times of it
+    {
+        const float m = wave_top(lim);
+        meet(m, m > 0.0f ? wave_count(m * 0.015625f, lim) : 0);
+#pragma unroll
+        for (int i = 0; i < XP_T / 64; ++i)
+            if (tops[0][i] > top) {
+                top = tops[0][i];
+                crowd = counts[0][i];
+            }
+    }
+    // no outliers where the top's own wave says so (most rows: no second scan)
+    for (int left = EX_OUT; crowd <= EX_OUT && top > 0.0f;) {
+        const float cut = top * 0.015625f;
+        turn ^= 1;
+        meet(wave_top(cut), wave_count(cut, lim));
+        float rest = 0.0f;
+        int count = 0;
+#pragma unroll
+        for (int i = 0; i < XP_T / 64; ++i) {
+            rest = fmaxf(rest, tops[turn][i]);
+            count += counts[turn][i];
+        }
+        if (count > left || rest == 0.0f) break;
+        left -= count;  // at least one
+        lim = cut;
+        top = rest;
+    }
+    const int e = top > 0.0f ? __builtin_amdgcn_frexp_expf(top) - 15 : 0;
+    if (tid == 0) E[row] = e;
 
-    auto emit = [&](int p, const float (&a)[8]) {
-        h8_t h0, h1;
-        float s = 0.0f, xs[8];
+    each([&](int p, const float (&a)[8]) {
+        h8_t h0, h1, h2;
+        float xs[8];
+        bool lost[8], any = false;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            xs[i] = fin ? ldexpf(a[i], -e) : 0.0f;
+            const bool in = fabsf(a[i]) < lim;
+            xs[i] = in ? __builtin_amdgcn_ldexpf(a[i], -e) : 0.0f;
             h0[i] = (_Float16)xs[i];
-            h1[i] = (_Float16)(xs[i] - (float)h0[i]);
+            const float r1 = (xs[i] - (float)h0[i]) * EX_UP;
+            h1[i] = (_Float16)r1;
+            const float r2 = r1 - (float)h1[i];
+            h2[i] = (_Float16)r2;
+            lost[i] = (float)h2[i] != r2 || (xs[i] == 0.0f && a[i] != 0.0f);  // not in, or too small
+            any |= lost[i];
+        }
+        if (any) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (!lost[i]) continue;
+                const int at = atomicAdd(&nlist, 1);
+                if (at < EX_LIST) list[at] = ExItem{8 * p + i, a[i]};
+                h0[i] = h1[i] = h2[i] = (_Float16)0.0f;
+                xs[i] = 0.0f;
+            }
         }
         P[(row * K >> 3) + p] = h0;
         P[((plane + row * K) >> 3) + p] = h1;
+        P[((2 * plane + row * K) >> 3) + p] = h2;
         if constexpr (QT == 12 || QT == 13) {
-            s = ((xs[0] + xs[1]) + (xs[2] + xs[3])) + ((xs[4] + xs[5]) + (xs[6] + xs[7]));
+            float s = ((xs[0] + xs[1]) + (xs[2] + xs[3])) + ((xs[4] + xs[5]) + (xs[6] + xs[7]));
             s = dpp_quad(s);  // 32 values (8-value pieces go to lanes in order; K % 256 == 0: whole waves' octets)
-            if constexpr (QT == 12) {
-                if ((p & 3) == 0) {
-                    const int j = p >> 2;
-                    const float ss = s * 0.015625f;
-                    const _Float16 s0 = (_Float16)ss;
-                    _Float16* d = SS + (row * (K >> 8) + (j >> 3)) * 16 + (j & 7);
-                    d[0] = s0;
-                    d[8] = (_Float16)(ss - (float)s0);
-                }
-            } else {
+            if constexpr (QT == 13)
                 s += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(s), 0x141, 0xF, 0xF, false));
-                if ((p & 7) == 0) SA[(int64_t)(p >> 3) * mpad + row] = s;
-            }
+            constexpr int W = QT == 13 ? 8 : 4;
+            if ((p & (W - 1)) == 0) SA[(int64_t)(p / W) * mpad + row] = s;
         }
-    };
-#pragma unroll
-    for (int j = 0; j < XP_KEEP; ++j) {
-        const int p = tid + j * XP_T;
-        if (p < n8) emit(p, v[j]);
-    }
-    for (int p = tid + XP_KEEP * XP_T; p < n8; p += XP_T) {
-        float a[8];
-        load8(x + 8 * p, a);
-        emit(p, a);
+    });
+    __syncthreads();
+    const int n = nlist;
+    if (tid == 0) LC[row] = n > EX_LIST ? -1 : n;
+    if (n <= EX_LIST && tid < n) {  // in ascending order, whoever came first
+        int rank = 0;
+        for (int i = 0; i < n; ++i) rank += list[i].k < list[tid].k;
+        LK[row * EX_LIST + rank] = list[tid];
     }
 }
 
@@ -234,25 +319,38 @@ template <>
 struct ExHalf<14> {
     ex_u32x2 ql[2][2], qh[2];
 };
+// the loads of R are waited for here
+template <int QT>
+__device__ __forceinline__ void ex_settle(ExHalf<QT>& R) {
+    if constexpr (QT == 14) {
+        asm volatile("" : "+v"(R.ql[0][0]), "+v"(R.ql[0][1]), "+v"(R.ql[1][0]), "+v"(R.ql[1][1]), "+v"(R.qh[0]),
+                     "+v"(R.qh[1]));
+    } else {
+        asm volatile("" : "+v"(R.w[0]), "+v"(R.w[1]));
+        if constexpr (QT == 8) asm volatile("" : "+v"(R.w[2]), "+v"(R.w[3]));
+    }
+}
 
+// R: activation rows per group (8, 16 or 32).
 // OUT: 0 = K-split partials f32 [split][M][nrows], 1 = f32, 2 = bf16
-template <int QT, bool ST, bool GU, int OUT>
+template <int QT, int R, bool GU, int OUT>
 __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uint8_t* Wa, const _Float16* P,
-                                                        const int* __restrict__ EX, const _Float16* SS,
-                                                        const float* SA, int64_t mpad, const float* X,
-                                                        void* __restrict__ Yv, int M, int K, int64_t nout,
-                                                        int64_t up_off, int64_t nrows, int cps, int tiles,
-                                                        int splits) {
-    constexpr int NW = 4;                      // waves
-    constexpr int NP = ST ? 1 : 2;             // operands per 32 rows
-    constexpr int MP = ST ? 16 : 32;           // activation rows per group
-    constexpr int VR = ST ? 32 : NP * MP;      // operand rows in LDS
-    constexpr int XB = VR * 512;               // bytes per buffer
-    constexpr int NJ = VR / (2 * NW);          // copy instructions per wave per chunk
-    constexpr int SR = 32;                     // rows of the affine sums in LDS
-    constexpr bool AFF = QT == 13;
-    __shared__ __attribute__((aligned(16))) uint8_t xs[2 * XB];
-    __shared__ float sas[AFF ? 2 * 4 * SR : 1];
+                                                        const int* __restrict__ EX, const int* __restrict__ LC,
+                                                        const ExItem* __restrict__ LK, const float* SA, int64_t mpad,
+                                                        const float* X, void* __restrict__ Yv, int M, int K,
+                                                        int64_t nout, int64_t up_off, int64_t nrows, int cps,
+                                                        int tiles, int splits) {
+    constexpr int NW = 4;                              // waves
+    constexpr int VR = R == 8 ? 32 : 3 * R;            // operand rows in LDS (R = 8: plane 2 twice)
+    constexpr int NP = (3 * R + 31) / 32;              // operands
+    constexpr int NA = R == 32 ? 1 : NP;               // accumulators per tile
+    constexpr int HB = VR * 256;                       // bytes per half chunk
+    constexpr int NJ = VR / (4 * NW);                  // copy instructions per wave per half chunk
+    constexpr int NSUM = QT == 12 ? 8 : QT == 13 ? 4 : 0;  // offset sums per chunk and row
+    constexpr float DOWN = 1.0f / EX_UP;
+    __shared__ __attribute__((aligned(16))) uint8_t xs[2 * HB];
+    __shared__ __attribute__((aligned(16))) float sas[NSUM ? 2 * NSUM * R : 1];
+    static_assert(2 * HB >= R * 64 * NW * 4, "the listed elements' products reuse xs");
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -270,8 +368,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
     const int nch = K >> 8;
     const int cb = split * cps;
     const int ce = cb + cps < nch ? cb + cps : nch;
-    const int m0 = group * MP;
-    const int Mz = M - m0 < MP ? M - m0 : MP;
+    const int m0 = group * R;
+    const int Mz = M - m0 < R ? M - m0 : R;
 
     int64_t orow[2], row[2];
     bool valid[2];
@@ -294,33 +392,34 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
             od[t] = (uint32_t)(L6.d + row[t] * (K / 256) * 2);
         } else {
             ow[t] = (uint32_t)q4k_piece(row[t], nch, 0, g, 0);
-            oh[t] = (uint32_t)q4k_hdword(row[t], nch, 0, 0);
+            oh[t] = (uint32_t)q4k_hdword(row[t], nch, 0, 2 * g);
         }
     }
-    auto wload = [&](ExHalf<QT> (&R)[2], int c, int hf) {
+    auto wload = [&](ExHalf<QT> (&H)[2], int c, int hf) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             if constexpr (QT == 8) {
                 const uint8_t* b = Wq + (int64_t)c * 8192 + hf * 4096;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) R[t].w[j] = *reinterpret_cast<const ex_u32x4*>(b + ow[t] + j * 1024);
+                for (int j = 0; j < 4; ++j) H[t].w[j] = *reinterpret_cast<const ex_u32x4*>(b + ow[t] + j * 1024);
             } else if constexpr (QT == 14) {
                 const uint8_t* b = Wq + (int64_t)c * 128 + hf * 64;
                 const uint8_t* bh = Wq + (int64_t)c * 64 + hf * 32;
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    R[t].ql[u][0] = *reinterpret_cast<const ex_u32x2*>(b + ow[t] + u * 32);
-                    R[t].ql[u][1] = *reinterpret_cast<const ex_u32x2*>(b + ow[t] + u * 32 + 16);
-                    R[t].qh[u] = *reinterpret_cast<const ex_u32x2*>(bh + oq[t] + u * 16);
+                    H[t].ql[u][0] = *reinterpret_cast<const ex_u32x2*>(b + ow[t] + u * 32);
+                    H[t].ql[u][1] = *reinterpret_cast<const ex_u32x2*>(b + ow[t] + u * 32 + 16);
+                    H[t].qh[u] = *reinterpret_cast<const ex_u32x2*>(bh + oq[t] + u * 16);
                 }
             } else {
                 const uint8_t* b = Wq + (int64_t)c * 64 + hf * 32;
-                R[t].w[0] = *reinterpret_cast<const ex_u32x4*>(b + ow[t]);
-                R[t].w[1] = *reinterpret_cast<const ex_u32x4*>(b + ow[t] + 16);
+                H[t].w[0] = *reinterpret_cast<const ex_u32x4*>(b + ow[t]);
+                H[t].w[1] = *reinterpret_cast<const ex_u32x4*>(b + ow[t] + 16);
             }
         }
     };
-    // a chunk's header: Q4_K / affine four dwords, Q8_0 eight f16 scales, Q6_K sixteen int8 scales (and d)
+    // a chunk's header: Q4_K / affine four dwords (loaded as two per lane half,
+    // h[0..1], and met in hmeet), Q8_0 eight f16 scales, Q6_K sixteen int8 scales (and d)
     struct Hdr {
         ex_u32x4 h;
         uint32_t d;
@@ -337,254 +436,307 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
             } else {
                 const uint8_t* b = Wq + (int64_t)c * 64;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) H[t].h[u] = *reinterpret_cast<const uint32_t*>(b + oh[t] + u * 16);
+                for (int u = 0; u < 2; ++u) H[t].h[u] = *reinterpret_cast<const uint32_t*>(b + oh[t] + u * 16);
             }
         }
     };
+    auto hmeet = [&](const Hdr& H) {
+        Hdr r = H;
+        if constexpr (QT == 12 || QT == 13) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const auto p = __builtin_amdgcn_permlane32_swap(H.h[u], H.h[u], false, false);
+                r.h[u] = p[0];  // lane half 0's on both
+                r.h[2 + u] = p[1];
+            }
+        }
+        return r;
+    };
 
-    // copy j of a wave fills operand rows 2 (wave + NW j) and the next; the
-    // 16-B piece p of row r sits at slot p ^ (r & 15); rows past the group copy its last
+    // copy j of a wave fills operand rows 4 (wave + NW j) .. + 3 of a half
+    // chunk; the 16-B piece p of row r sits at slot p ^ (r & 15); rows past the
+    // group copy its last
     uint32_t xoff[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const int r = 2 * (wave + NW * j) + (lane >> 5);
-        const int pl = r / MP, rr = r % MP < Mz ? r % MP : Mz - 1;
-        xoff[j] = ((uint32_t)(pl * M + m0 + rr) * (uint32_t)K) * 2u + 16u * (uint32_t)((lane & 31) ^ (r & 15));
+        const int r = 4 * (wave + NW * j) + (lane >> 4);
+        const int pl = r / R < 3 ? r / R : 2, rr = r % R < Mz ? r % R : Mz - 1;
+        xoff[j] = ((uint32_t)(pl * M + m0 + rr) * (uint32_t)K) * 2u + 16u * (uint32_t)((lane & 15) ^ (r & 15));
     }
     const uint32_t xs0 = ex_lds(xs);
-    auto xcopy = [&](int c, int b) {
-        const uint8_t* xc = reinterpret_cast<const uint8_t*>(P) + (int64_t)c * 512;
+    auto xcopy = [&](int h, int b) {  // half chunk h into buffer b
+        const uint8_t* xc = reinterpret_cast<const uint8_t*>(P) + (int64_t)h * 256;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-            ex_dma16(__builtin_amdgcn_readfirstlane(xs0 + (uint32_t)(b * XB + (wave + NW * j) * 1024)), xc, xoff[j]);
+            ex_dma16(__builtin_amdgcn_readfirstlane(xs0 + (uint32_t)(b * HB + (wave + NW * j) * 1024)), xc, xoff[j]);
     };
-    auto aread = [&](const uint8_t* xb, int pl, int u, int k) {
-        const int p = QT == 14 ? 8 * u + 2 * k + g : 8 * u + 2 * g + (k & 1) + 4 * (k >> 1);
-        return *reinterpret_cast<const h8_t*>(xb + (pl * MP + n) * 512 + 16 * (p ^ (n & 15)));
+    auto aread = [&](int b, int op, int up, int k) {
+        const int r = R == 16 && op ? 32 + (n & 15) : 32 * op + n;  // R = 16: plane 2 twice
+        const int p = QT == 14 ? 8 * up + 2 * k + g : 8 * up + 2 * g + (k & 1) + 4 * (k >> 1);
+        return *reinterpret_cast<const h8_t*>(xs + b * HB + r * 256 + 16 * (p ^ (n & 15)));
     };
-    // affine sums of chunk c: thread tid holds (64-wide part tid / SR, row tid % SR)
+    // offset sums of chunk c: thread tid holds (piece tid / R, row tid % R)
     auto sload = [&](int c) {
-        if constexpr (!AFF) return 0.0f;
-        const int tid = threadIdx.x & (4 * SR - 1), r = tid % SR;
-        const float v = SA[(int64_t)(4 * c + tid / SR) * mpad + m0 + (r < Mz ? r : 0)];
+        if constexpr (!NSUM) return 0.0f;
+        const int tid = threadIdx.x & (NSUM * R - 1), r = tid % R;
+        const float v = SA[(int64_t)(NSUM * c + tid / R) * mpad + m0 + (r < Mz ? r : 0)];
         return r < Mz ? v : 0.0f;
     };
     auto sstore = [&](float v, int b) {
-        if constexpr (AFF) sas[b * 4 * SR + (threadIdx.x & (4 * SR - 1))] = v;
+        if constexpr (NSUM) sas[b * NSUM * R + (threadIdx.x & (NSUM * R - 1))] = v;
     };
-
-    f32x16_t acc[2];
+    f32x16_t acc[2][NA];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) acc[t] = f32x16_t{};
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) acc[t][i] = f32x16_t{};
 
-    // one 64-wide part u (0..3) of the chunk in LDS buffer b
-    auto part = [&](const ExHalf<QT> (&R)[2], const Hdr (&H)[2], const float (&d)[2], int u, int b) {
+    // part u (0..3) of a chunk, in half buffer b
+    auto part = [&](const ExHalf<QT> (&W)[2], const Hdr (&H)[2], const float (&d)[2], int u, int b) {
         constexpr int SEG = QT == 14 ? 1 : (QT == 8 ? 2 : 4);  // 16-wide steps per scale
         constexpr int NSEG = 4 / SEG;
-        const uint8_t* xb = xs + b * XB;
+        constexpr bool SUM = NSEG > 1;  // a part's sum is added to acc once
         const uint32_t M4 = 0x0F0F0F0Fu;
         const int up = u & 1;
-        h8_t B[2][4];
-        float ds[2][NSEG];
+        constexpr bool TILES = !(R == 16 && NSEG > 1);  // tiles inside a scale's steps share A; else T would be 64 registers
+        f32x16_t T[2][NA];
+        h8_t A[NP][SEG];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int q = 0; q < 2 * NSEG; ++q) {
+            const int t = TILES ? q & 1 : q / NSEG, sg = TILES ? q >> 1 : q % NSEG;
+            if (!TILES || t == 0) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+                for (int op = 0; op < NP; ++op)
+#pragma unroll
+                    for (int k = 0; k < SEG; ++k) A[op][k] = aread(b, op, up, SEG * sg + k);
+            }
+            h8_t B[SEG];
+#pragma unroll
+            for (int i = 0; i < SEG; ++i) {
+                const int k = SEG * sg + i;
                 if constexpr (QT == 8) {
-                    const ex_u32x4 q = R[t].w[2 * up + (k >> 1)] ^ 0x80808080u;
-                    B[t][k] = ex_codes(q[2 * (k & 1)], q[2 * (k & 1) + 1], (_Float16)128.0f);
+                    const ex_u32x4 w = W[t].w[2 * up + (k >> 1)] ^ 0x80808080u;
+                    B[i] = ex_codes(w[2 * (k & 1)], w[2 * (k & 1) + 1], (_Float16)128.0f);
                 } else if constexpr (QT == 14) {
-                    const ex_u32x2 ql = R[t].ql[up][k & 1], qh = R[t].qh[up];
+                    const ex_u32x2 ql = W[t].ql[up][k & 1], qh = W[t].qh[up];
                     uint32_t c[2];
 #pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        c[i] = ((ql[i] >> (4 * (k >> 1))) & M4) | (((qh[i] >> (2 * k)) & 0x03030303u) << 4);
-                    B[t][k] = ex_codes(c[0], c[1], (_Float16)32.0f);
+                    for (int j = 0; j < 2; ++j)
+                        c[j] = ((ql[j] >> (4 * (k >> 1))) & M4) | (((qh[j] >> (2 * k)) & 0x03030303u) << 4);
+                    B[i] = ex_codes(c[0], c[1], (_Float16)32.0f);
                 } else {
-                    const ex_u32x4 q = R[t].w[up];
-                    const int sh = k < 2 ? 0 : 4, i = 2 * (k & 1);
-                    B[t][k] = ex_codes((q[i] >> sh) & M4, (q[i + 1] >> sh) & M4, (_Float16)8.0f);
-                    if constexpr (QT == 12) B[t][k] *= (_Float16)(uint16_t)((H[t].h[u] >> (k < 2 ? 0 : 12)) & 63u);
+                    const ex_u32x4 w = W[t].w[up];
+                    const int sh = k < 2 ? 0 : 4, c = 2 * (k & 1);
+                    B[i] = ex_codes((w[c] >> sh) & M4, (w[c + 1] >> sh) & M4, (_Float16)8.0f);
+                    if constexpr (QT == 12) B[i] *= (_Float16)(uint16_t)((H[t].h[u] >> (k < 2 ? 0 : 12)) & 63u);
                 }
             }
-#pragma unroll
-            for (int sg = 0; sg < NSEG; ++sg) {
-                if constexpr (QT == 8) {
-                    ds[t][sg] = f16_to_f32((uint16_t)(sg ? H[t].h[u] >> 16 : H[t].h[u]));
-                } else if constexpr (QT == 14) {
-                    ds[t][sg] = d[t] * (float)(int8_t)(H[t].h[u] >> (8 * sg));
-                } else {
-                    ds[t][sg] = QT == 12 ? d[t] : aff_scale(H[t].h[u]);
-                }
-            }
-        }
-        h8_t A[NP][4];
-#pragma unroll
-        for (int pl = 0; pl < NP; ++pl)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) A[pl][k] = aread(xb, pl, u, k);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            f32x16_t T;  // the part's sum, added to acc once
-#pragma unroll
-            for (int sg = 0; sg < NSEG; ++sg) {
-                f32x16_t D = {}, D1 = {};
+            float ds;
+            if constexpr (QT == 8)
+                ds = f16_to_f32((uint16_t)(sg ? H[t].h[u] >> 16 : H[t].h[u]));
+            else if constexpr (QT == 14)
+                ds = d[t] * (float)(int8_t)(H[t].h[u] >> (8 * sg));
+            else
+                ds = QT == 12 ? d[t] : aff_scale(H[t].h[u]);
+            f32x16_t D[NP == 3 ? 2 : NP] = {};
+            if constexpr (R == 32) {  // plane 0, and planes 1 and 2 together
 #pragma unroll
                 for (int k = 0; k < SEG; ++k) {
-                    if constexpr (NP == 2) D1 = ex_mfma(A[1][SEG * sg + k], B[t][SEG * sg + k], D1);
-                    D = ex_mfma(A[0][SEG * sg + k], B[t][SEG * sg + k], D);
+                    D[1] = ex_mfma(A[1][k], B[k], D[1]);
+                    D[0] = ex_mfma(A[0][k], B[k], D[0]);
+                    D[1] = ex_mfma(A[2][k], B[k], D[1]);
                 }
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float v = NP == 2 ? D[e] + D1[e] : D[e];
-                    if constexpr (NSEG == 1 && !AFF)
-                        acc[t][e] = __builtin_fmaf(ds[t][0], v, acc[t][e]);
-                    else
-                        T[e] = sg ? __builtin_fmaf(ds[t][sg], v, T[e]) : ds[t][0] * v;
-                }
+                for (int e = 0; e < 16; ++e) D[0][e] = __builtin_fmaf(DOWN, D[1][e], D[0][e]);
+            } else {
+#pragma unroll
+                for (int op = 0; op < NP; ++op)
+#pragma unroll
+                    for (int k = 0; k < SEG; ++k) D[op] = ex_mfma(A[op][k], B[k], D[op]);
             }
-            if constexpr (AFF) {
-                // (bias + 8 scale) x the part's sum of each row
-                const float cf = __builtin_fmaf(8.0f, ds[t][0], aff_bias(H[t].h[u]));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const f32x4_t v =
-                        *reinterpret_cast<const f32x4_t*>(&sas[(b * 4 + u) * SR + 8 * i + 4 * g]);
+            for (int a = 0; a < NA; ++a) {
+                f32x16_t& S = SUM ? T[t][a] : acc[t][a];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) T[4 * i + e] = __builtin_fmaf(cf, v[e], T[4 * i + e]);
-                }
-            }
-            if constexpr (NSEG > 1 || AFF) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[t][e] += T[e];
+                for (int e = 0; e < 16; ++e) S[e] = SUM && sg == 0 ? ds * D[a][e] : __builtin_fmaf(ds, D[a][e], S[e]);
+                asm volatile("" : "+v"(S));  // now: left to the end, every D stays live
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (SUM) {
+                if (sg != NSEG - 1) continue;
+#pragma unroll
+                for (int a = 0; a < NA; ++a) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[t][a][e] += T[t][a][e];
+                    asm volatile("" : "+v"(acc[t][a]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);
     };
-    // Q4_K: sum_j c_j S_j of a chunk, c_j = 8 d sc_j - dmin m_j: two MFMAs per
-    // tile, the sums' two pieces (lane half g holds piece g) by c_j's two, c
-    // scaled by a power of two into f16's range.  (As 8 d sum sc_j S_j - dmin
-    // sum m_j S_j the two large sums' roundings add 1e-7.)
-    auto offsets = [&](const Hdr (&H)[2], const float (&d)[2], const float (&dm)[2], const h8_t& As) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            float cj[8], mx = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t w = H[t].h[j >> 1] >> (12 * (j & 1));
-                cj[j] = __builtin_fmaf(8.0f * d[t], (float)(w & 63u), -(dm[t] * (float)((w >> 6) & 63u)));
-                mx = fmaxf(mx, fabsf(cj[j]));
-            }
-            const int ce_ = __builtin_amdgcn_frexp_expf(mx) - 14;
-            const float up = __builtin_amdgcn_ldexpf(1.0f, -ce_), down = __builtin_amdgcn_ldexpf(64.0f, ce_);
-            h8_t C0, C1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = cj[j] * up;
-                C0[j] = (_Float16)v;
-                C1[j] = (_Float16)(v - (float)C0[j]);
-            }
-            const f32x16_t a = ex_mfma(As, C0, ex_mfma(As, C1, f32x16_t{}));
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[t][e] = __builtin_fmaf(down, a[e], acc[t][e]);
+    // 4-bit weights: sum_j c_j S_j of a chunk, added to acc once.  Q4_K: c_j =
+    // 8 d sc_j - dmin m_j (as 8 d sum sc_j S_j - dmin sum m_j S_j the two large
+    // sums' roundings add 1e-7), affine: c_j = 8 scale_j + bias_j.
+    auto offset = [&](const Hdr& H, float d, float dm, int j, int half) {  // c_{j + half}, j even
+        if constexpr (QT == 12) {
+            const uint32_t w = H.h[j >> 1] >> (12 * half);
+            return __builtin_fmaf(8.0f * d, (float)(w & 63u), -(dm * (float)((w >> 6) & 63u)));
         }
+        const uint32_t w = half ? H.h[(j + 1) & 3] : H.h[j & 3];
+        return __builtin_fmaf(8.0f, aff_scale(w), aff_bias(w));
+    };
+    auto offsets = [&](const Hdr (&H)[2], const float (&d)[2], const float (&dm)[2], int sb) {
+        f32x16_t T[2] = {};
+        if constexpr (R == 32) {  // on the f32 matrix cores: lane half g holds j + g
+#pragma unroll
+            for (int j = 0; j < NSUM; j += 2) {
+                const float v = sas[(sb * NSUM + j + g) * R + n];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    T[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, offset(H[t], d[t], dm[t], j, g), T[t], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NSUM; ++j) {
+                const float c[2] = {offset(H[0], d[0], dm[0], j & ~1, j & 1), offset(H[1], d[1], dm[1], j & ~1, j & 1)};
+#pragma unroll
+                for (int i = 0; i < R / 8; ++i) {
+                    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sas[(sb * NSUM + j) * R + 8 * i + 4 * g]);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) T[t][4 * i + e] = __builtin_fmaf(c[t], v[e], T[t][4 * i + e]);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < R / 2; ++e) acc[t][0][e] += T[t][e];
     };
 
-    ExHalf<QT> R0[2], R1[2];
+    ExHalf<QT> W[2][2];
     Hdr Hc[2], Hn[2];
     auto last = [&](int c) { return c < ce ? c : ce - 1; };
-    xcopy(cb, 0);
+    xcopy(2 * cb, 0);
     hload(Hn, cb);
-    wload(R0, cb, 0);
-    wload(R1, cb, 1);
+    wload(W[0], cb, 0);
+    wload(W[1], cb, 1);
     sstore(sload(cb), 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    // step c (buffer b): chunk c + 1's copies go out first (buffer b ^ 1, read
-    // by no wave since the last barrier); each half's weights are loaded again
-    // for chunk c + 1 as soon as it is consumed and stay in flight across the
-    // barrier: loads complete in order and the first half's and the header's
-    // are ten or more instructions behind the copies, so vmcnt(10) waits for
-    // the copies only.  Past the range they repeat the last chunk.
+    // Half hf of chunk c computes from buffer hf while the next half's copies
+    // go into the other one, read by no wave since the last barrier.  Its own
+    // weights are settled before the copies go out (a wait for them behind the
+    // copies, which the compiler does not count, would wait for the copies
+    // too); the next chunk's are loaded into the same registers at its end and
+    // stay in flight across the barrier, for the whole of the next half: its
+    // vmcnt(0) is for them and for its copies.  Past the range they repeat the
+    // last chunk.
     for (int c = cb; c < ce; ++c) {
-        const int b = (c - cb) & 1;
-        float d[2], dm[2];
+        const int sb = (c - cb) & 1;
+        float d[2], dm[2], sn = 0.0f;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            Hc[t] = Hn[t];
-            d[t] = dm[t] = 0.0f;
-            if constexpr (QT == 12) {
-                d[t] = f16_to_f32((uint16_t)__builtin_amdgcn_perm(Hc[t].h[1], Hc[t].h[0], 0x0c0c0703u));
-                dm[t] = f16_to_f32((uint16_t)__builtin_amdgcn_perm(Hc[t].h[3], Hc[t].h[2], 0x0c0c0703u));
+        for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) ex_settle<QT>(W[hf][t]);
+            if (hf == 0) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    if constexpr (QT == 8 || QT == 14)
+                        asm volatile("" : "+v"(Hn[t].h), "+v"(Hn[t].d));
+                    else
+                        asm volatile("" : "+v"(Hn[t].h[0]), "+v"(Hn[t].h[1]));
+                    Hc[t] = hmeet(Hn[t]);
+                    d[t] = dm[t] = 0.0f;
+                    if constexpr (QT == 12) {
+                        d[t] = f16_to_f32((uint16_t)__builtin_amdgcn_perm(Hc[t].h[1], Hc[t].h[0], 0x0c0c0703u));
+                        dm[t] = f16_to_f32((uint16_t)__builtin_amdgcn_perm(Hc[t].h[3], Hc[t].h[2], 0x0c0c0703u));
+                    }
+                    if constexpr (QT == 14) d[t] = f16_to_f32((uint16_t)Hc[t].d);
+                }
+            } else {
+                sn = sload(last(c + 1));
             }
-            if constexpr (QT == 14) d[t] = f16_to_f32((uint16_t)Hc[t].d);
+            __builtin_amdgcn_sched_barrier(0);
+            const int next = 2 * c + hf + 1;
+            xcopy(next < 2 * ce ? next : 2 * ce - 1, hf ^ 1);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            part(W[hf], Hc, d, 2 * hf, hf);
+            part(W[hf], Hc, d, 2 * hf + 1, hf);
+            if constexpr (NSUM)
+                if (hf) offsets(Hc, d, dm, sb);
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (hf) sstore(sn, sb ^ 1);
+            wload(W[hf], last(c + 1), hf);
+            if (hf == 0) hload(Hn, last(c + 1));
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
         }
-        xcopy(last(c + 1), b ^ 1);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        const float sn = sload(last(c + 1));
-        h8_t As = {};
-        if constexpr (QT == 12) {
-            As = *reinterpret_cast<const h8_t*>(SS + (((int64_t)(m0 + (n < Mz ? n : 0)) * nch + c) * 2 + g) * 8);
-            if (n >= Mz) As = h8_t{};
-        }
-        part(R0, Hc, d, 0, b);
-        part(R0, Hc, d, 1, b);
-        __builtin_amdgcn_sched_barrier(0);
-        wload(R0, last(c + 1), 0);
-        hload(Hn, last(c + 1));
-        __builtin_amdgcn_sched_barrier(0);
-        part(R1, Hc, d, 2, b);
-        part(R1, Hc, d, 3, b);
-        if constexpr (QT == 12) offsets(Hc, d, dm, As);
-        sstore(sn, b ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
-        wload(R1, last(c + 1), 1);
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
     }
 
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may land in LDS after the block ends
-    // epilogue: acc[t][e] is operand row 8 (e / 4) + 4 g + e % 4
-    auto put = [&](int m, int t, float v, float vu) {
-        if constexpr (OUT == 0) {
-            static_cast<float*>(Yv)[((int64_t)split * M + m0 + m) * nrows + row[t]] = v;
-        } else {
-            using YT = std::conditional_t<OUT == 1, float, bf16_t>;
-            store_y<YT>(static_cast<YT*>(Yv) + (int64_t)(m0 + m) * nout + orow[t], GU ? silu_mul(v, vu) : v);
-        }
+    // acc[t][a][e] is operand row 8 (e / 4) + 4 g + e % 4; a row's value
+    auto value = [&](int t, int e) {
+        if constexpr (R == 32) return acc[t][0][e];
+        if constexpr (R == 16) return __builtin_fmaf(DOWN, acc[t][0][(e + 8) & 15] + acc[t][NA - 1][e], acc[t][0][e]);
+        return __builtin_fmaf(DOWN, acc[t][0][(e + 4) & 15] + acc[t][0][(e + 8) & 15], acc[t][0][e]);
     };
     constexpr int NT = GU && OUT != 0 ? 1 : 2;  // stored tiles (gate/up: one, the gate's)
+    // the rows with listed elements, and of those the ones dotted whole: f32
+    // dots over the split's K into LDS (lane half g takes every other element)
+    const int lc = lane < Mz ? LC[m0 + lane] : 0;
+    const uint32_t some = (uint32_t)__ballot(lc != 0), whole = (uint32_t)__ballot(lc < 0);
+    float* const side = reinterpret_cast<float*>(xs) + wave * 64 + n;  // [row][wave][t][n], no copy in flight
+    for (uint32_t left = some; left; left &= left - 1) {
+        const int m = __builtin_ctz(left);
+        const bool all = (whole >> m) & 1;
+        const int cnt = all ? (ce - cb) * 256 : __builtin_amdgcn_readlane(lc, m);
+        float v[2] = {0.0f, 0.0f};
+#pragma clang loop unroll(disable)
+        for (int i = g; i < cnt; i += 2) {
+            ExItem it;
+            if (all) {
+                it.k = cb * 256 + i;
+                it.x = load_x<float>(X + (int64_t)(m0 + m) * K + it.k);
+            } else {
+                it = LK[(int64_t)(m0 + m) * EX_LIST + i];
+                if (it.k < cb * 256 || it.k >= ce * 256) continue;
+            }
 #pragma unroll
-    for (int e = 0; e < (ST ? 8 : 16); ++e) {
+            for (int t = 0; t < 2; ++t)
+                v[t] = __builtin_fmaf(it.x, ex_weight<QT>(Wq, Wa, row[t], K, nrows, it.k), v[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) side[m * 64 * NW + 32 * t] = v[t] + __shfl_xor(v[t], 32, 64);
+    }
+#pragma unroll
+    for (int e = 0; e < R / 2; ++e) {
         const int m = 8 * (e >> 2) + 4 * g + (e & 3);
         if (m >= Mz) continue;
         const int ex = EX[m0 + m];
-        if (ex == EX_NONFINITE) continue;
         float v[2];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) v[t] = ldexpf(ST ? acc[t][e] + acc[t][(e + 8) & 15] : acc[t][e], ex);
+        for (int t = 0; t < 2; ++t) v[t] = ldexpf(value(t, e), ex);
+        if ((some >> m) & 1) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
-            if (valid[t]) put(m, t, v[t], v[1]);
-    }
-    // rows with Inf / NaN: f32 dots over the split's K (lane half g takes every other column)
-    for (int m = 0; m < Mz; ++m) {
-        if (EX[m0 + m] != EX_NONFINITE) continue;
-        float v[2] = {0.0f, 0.0f};
-#pragma clang loop unroll(disable)
-        for (int k = cb * 256 + g; k < ce * 256; k += 2) {
-            const float x = load_x<float>(X + (int64_t)(m0 + m) * K + k);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) v[t] = __builtin_fmaf(x, ex_weight<QT>(Wq, Wa, row[t], K, nrows, k), v[t]);
+            for (int t = 0; t < 2; ++t) {
+                const float f = side[m * 64 * NW + 32 * t];
+                v[t] = (whole >> m) & 1 ? f : v[t] + f;
+            }
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) v[t] += __shfl_xor(v[t], 32, 64);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-            if (g == 0 && valid[t]) put(m, t, v[t], v[1]);
+        for (int t = 0; t < NT; ++t) {
+            if (!valid[t]) continue;
+            if constexpr (OUT == 0) {
+                static_cast<float*>(Yv)[((int64_t)split * M + m0 + m) * nrows + row[t]] = v[t];
+            } else {
+                using YT = std::conditional_t<OUT == 1, float, bf16_t>;
+                store_y<YT>(static_cast<YT*>(Yv) + (int64_t)(m0 + m) * nout + orow[t],
+                            GU ? silu_mul(v[0], v[1]) : v[t]);
+            }
+        }
     }
 }
 
@@ -639,20 +791,32 @@ hipError_t ex_reduce(const float* P, YT* y, int M, int64_t nout, int64_t up_off,
 
 struct ExBufs {
     _Float16* P;
-    int* E;
-    _Float16* SS;
-    float* SA;
-    float* part;
+    int *E, *LC;
+    ExItem* LK;
+    float *SA, *part;
 };
 size_t ex_align(size_t b) { return (b + 255) & ~(size_t)255; }
-size_t ex_planes_bytes(int64_t M, int64_t K) { return ex_align((size_t)M * K * 4); }
-size_t ex_sums_bytes(int qtype, int64_t M, int64_t K) {
-    if (qtype == 12) return ex_align((size_t)M * (K / 256) * 32);
-    if (qtype == 13) return ex_align((size_t)(K / 64) * ((M + 63) / 64 * 64) * 4);
-    return 0;
+// the buffers of a call at `base`, and the bytes of all but the partials
+ExBufs ex_bufs(int qtype, int64_t M, int64_t K, void* base, size_t& bytes) {
+    char* q = static_cast<char*>(base);
+    auto take = [&](size_t n) {
+        char* at = q;
+        q += ex_align(n);
+        return at;
+    };
+    ExBufs b;
+    b.P = reinterpret_cast<_Float16*>(take((size_t)M * K * 6));
+    b.E = reinterpret_cast<int*>(take((size_t)M * 4));
+    b.LC = reinterpret_cast<int*>(take((size_t)M * 4));
+    b.LK = reinterpret_cast<ExItem*>(take((size_t)M * EX_LIST * sizeof(ExItem)));
+    const int64_t pieces = qtype == 12 ? K / 32 : qtype == 13 ? K / 64 : 0;
+    b.SA = reinterpret_cast<float*>(take((size_t)pieces * ((M + 63) / 64 * 64) * 4));
+    b.part = reinterpret_cast<float*>(q);
+    bytes = (size_t)(q - static_cast<char*>(base));
+    return b;
 }
 
-template <int QT, bool ST, bool GU>
+template <int QT, int R, bool GU>
 hipError_t run_ex(const ExPlan& p, const WeightView& w, const float* x, const ExBufs& b, void* y, bool yf32, int M,
                   int64_t nout, int64_t up_off, hipStream_t s) {
     const int64_t per = GU ? 128 : 256;
@@ -661,14 +825,15 @@ hipError_t run_ex(const ExPlan& p, const WeightView& w, const float* x, const Ex
     if (nb > 0x7FFFFFFF) return hipErrorInvalidValue;
     const int K = (int)w.K;
     const int64_t mpad = (int64_t)(M + 63) / 64 * 64;
-    hipLaunchKernelGGL((k_xplanes<QT>), dim3(M), dim3(XP_T), 0, s, x, K, (int64_t)M * K, reinterpret_cast<h8_t*>(b.P),
-                       b.E, b.SS, b.SA, mpad);
+    const auto planes = K <= 4096 ? k_xplanes<QT, 512, 1> : k_xplanes<QT, 1024, 2>;
+    hipLaunchKernelGGL(planes, dim3(M), dim3(K <= 4096 ? 512 : 1024), 0, s, x, K, (int64_t)M * K,
+                       reinterpret_cast<h8_t*>(b.P), b.E, b.LC, b.LK, b.SA, mpad);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 grid((unsigned)nb), block(256);
-#define THQ_EX(OUT_, Y_)                                                                                         \
-    hipLaunchKernelGGL((k_gemm_ex<QT, ST, GU, OUT_>), grid, block, 0, s, w.q, w.aux, b.P, b.E, b.SS, b.SA, mpad, x, \
-                       Y_, M, K, nout, up_off, w.N, p.cps, (int)tiles, p.splits)
+#define THQ_EX(OUT_, Y_)                                                                                              \
+    hipLaunchKernelGGL((k_gemm_ex<QT, R, GU, OUT_>), grid, block, 0, s, w.q, w.aux, b.P, b.E, b.LC, b.LK, b.SA, mpad, \
+                       x, Y_, M, K, nout, up_off, w.N, p.cps, (int)tiles, p.splits)
     if (p.splits > 1) {
         THQ_EX(0, (void*)b.part);
         e = hipGetLastError();
@@ -703,20 +868,20 @@ ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus
     const uint64_t plane = qtype == 8 ? (uint64_t)q8t_q_bytes(N, K)
                                       : (qtype == 14 ? (uint64_t)q6k_layout(N, K).total
                                                      : (uint64_t)((N + 3) / 4) * (uint64_t)(K / 256) * 576u);
-    if (plane >= lim || (uint64_t)M * (uint64_t)K * 4u >= lim) return p;
+    if (plane >= lim || (uint64_t)M * (uint64_t)K * 6u >= lim) return p;
     // Two blocks per CU.  Cost of a K split count: rounds of resident blocks
     // x chunks (and one of prologue) x a chunk's time (2.4 us stacked, 4.0 us
-    // with two operands), plus the partials' round trip at 4 TB/s.
+    // with 32 rows), plus the partials' round trip at 4 TB/s.
     const int64_t nch = K / 256, nout = gu ? N / 2 : N, cu = cus > 0 ? cus : 256;
-    p.stacked = M <= 16;
-    p.groups = (int)((M + (p.stacked ? 15 : 31)) / (p.stacked ? 16 : 32));
+    p.rows = M <= 8 ? 8 : M <= 16 ? 16 : 32;
+    p.groups = (int)((M + p.rows - 1) / p.rows);
     const int64_t per = gu ? 128 : 256, tiles = (nout + per - 1) / per;
     const int64_t smin = (nch + EX_CPS - 1) / EX_CPS;
     double best = 1e30;
     for (int64_t s = smin; s <= nch && s <= smin + 32; ++s) {
         const int64_t cps = (nch + s - 1) / s;
         const int64_t rounds = (tiles * p.groups * s + 2 * cu - 1) / (2 * cu);
-        const double t = (double)rounds * ((double)cps + 1.0) * (p.stacked ? 2.4 : 4.0) +
+        const double t = (double)rounds * ((double)cps + 1.0) * (p.rows < 32 ? 2.4 : 4.0) +
                          (s > 1 ? 2.0 + (double)s * (double)M * (double)N * 8.0 / 4.0e6 : 0.0);
         if (t < best - 1e-9) {
             best = t;
@@ -724,28 +889,20 @@ ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus
             p.splits = (int)((nch + cps - 1) / cps);
         }
     }
-    p.workspace_bytes = ex_planes_bytes(M, K) + ex_align((size_t)M * 4) + ex_sums_bytes(qtype, M, K) +
-                        (p.splits > 1 ? (size_t)p.splits * (size_t)M * (size_t)N * 4u : 0);
+    (void)ex_bufs(qtype, M, K, nullptr, p.workspace_bytes);
+    if (p.splits > 1) p.workspace_bytes += (size_t)p.splits * (size_t)M * (size_t)N * 4u;
     return p;
 }
 
 hipError_t launch_gemm_ex(const ExPlan& p, const WeightView& w, const float* x, void* y, bool yf32, bool gu, int M,
                           int64_t nout, int64_t up_off, void* ws, hipStream_t s) {
     if (p.groups < 1 || p.splits < 1 || M < 1 || !ws) return hipErrorInvalidValue;
-    char* q = static_cast<char*>(ws);
-    ExBufs b{};
-    b.P = reinterpret_cast<_Float16*>(q);
-    q += ex_planes_bytes(M, w.K);
-    b.E = reinterpret_cast<int*>(q);
-    q += ex_align((size_t)M * 4);
-    b.SS = reinterpret_cast<_Float16*>(q);
-    b.SA = reinterpret_cast<float*>(q);
-    q += ex_sums_bytes(w.qtype, M, w.K);
-    b.part = reinterpret_cast<float*>(q);
-#define THQ_EXG(QT_, ST_)                                                            \
-    (gu ? run_ex<QT_, ST_, true>(p, w, x, b, y, yf32, M, nout, up_off, s)            \
-        : run_ex<QT_, ST_, false>(p, w, x, b, y, yf32, M, nout, up_off, s))
-#define THQ_EXQ(QT_) (p.stacked ? THQ_EXG(QT_, true) : THQ_EXG(QT_, false))
+    size_t bytes;
+    const ExBufs b = ex_bufs(w.qtype, M, w.K, ws, bytes);
+#define THQ_EXG(QT_, R_)                                                           \
+    (gu ? run_ex<QT_, R_, true>(p, w, x, b, y, yf32, M, nout, up_off, s)           \
+        : run_ex<QT_, R_, false>(p, w, x, b, y, yf32, M, nout, up_off, s))
+#define THQ_EXQ(QT_) (p.rows == 8 ? THQ_EXG(QT_, 8) : p.rows == 16 ? THQ_EXG(QT_, 16) : THQ_EXG(QT_, 32))
     switch (w.qtype) {
         case 8: return THQ_EXQ(8);
         case 12: return THQ_EXQ(12);

@@ -174,7 +174,7 @@ hipError_t launch_gemm_rq(const RqPlan& p, bool affine, const uint8_t* wq, const
 // on row-scaled f16 activation planes (k_gemm_ex.hip); the workspace holds
 // the planes, then the split partials
 struct ExPlan {
-    bool stacked = false;     // up to 16 rows, both planes in one operand
+    int rows = 0;             // activation rows per group (8, 16 or 32)
     int groups = 0;           // row groups (0: unsupported)
     int splits = 0, cps = 0;  // K splits, 256-wide chunks per split
     size_t workspace_bytes = 0;
