@@ -51,18 +51,24 @@ def test_matches_row_tiles(qt, m, n, k, monkeypatch):
     assert torch.equal(q.matmul(w, torch.float32), y)
 
 
-@pytest.mark.parametrize("sign", [1.0, -1.0])
-def test_largest_integers(sign, monkeypatch):
-    """All nibbles 15, all scales and minima 63, all quants -128 (or 127): the largest sums the planes can reach."""
+@pytest.mark.parametrize("rest,quant", [(1.0, -128), (0.999, -128), (-0.999, 127)])
+def test_largest_integers(rest, quant, monkeypatch):
+    """All nibbles 15, all scales and minima 63, and rows whose quants are all -128 (a block's largest value always is;
+    the rest of its sign too) or, past the largest, 127: the largest sums of either sign that the planes can reach."""
     n, k, m = 64, 512, 40
     blk = np.zeros((n, k // 256, 144), np.uint8)
     blk[:, :, 0:4] = np.array([1.0, 0.5], np.float16).view(np.uint8)
     blk[:, :, 4:] = 0xFF
     w = thq.QTensor.from_gguf_bytes(O.Q4_K, blk.reshape(n, -1), n, k)
-    x = torch.full((m, k), sign, device="cuda")
-    x[:, ::256] = -sign * 1.001  # the block's largest: -128 of the other sign
+    x = torch.full((m, k), rest, device="cuda")
+    x[:, ::256] = 1.0
+    codes = thq.quantize_act(x, thq.Q8_K).view(m, k // 256, 292)[:, :, 4:260].contiguous().view(torch.int8)
+    assert (codes[:, :, 0] == -128).all() and (codes[:, :, 1:] == quant).all()
     ref, y = both(monkeypatch, lambda: thq.matmul(w, x, torch.float32, thq.MODE_Q8ACT))
     assert rel(y, ref) <= 4e-7
+    s = codes.double().sum(-1).sum(-1) * codes.new_tensor(-1.0 / 128, dtype=torch.float64)  # d = 1 / iscale = -1 / 128
+    exact = (63.0 * 15 - 0.5 * 63) * s  # d sc q - dmin m of every weight
+    assert rel(y, exact[:, None].expand(m, n)) <= 4e-7
 
 
 @pytest.mark.parametrize("qt", [O.Q4_K, O.Q8_0])
