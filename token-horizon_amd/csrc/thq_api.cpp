@@ -949,8 +949,22 @@ int exec_route(const Call& c, const Route& r, void* scratch, uint32_t* cnt = nul
     return THQ_OK;
 }
 
+// The workspace for a planned route behind `head` bytes, and for `tail` bytes
+// that follow the route in its place (caller holds ctx->mu).  Where it cannot
+// be had for the matrix-core routes of f32 rows and of THQ_MODE_Q8ACT, the
+// call is planned again without them: what ran there before needs less.
+int ensure_route(Call& c, Route& r, size_t head = 0, size_t tail = 0) {
+    int rc = ensure_ws(c.ctx, head + std::max(r.scratch, tail));
+    if (rc && (r.kind == Kind::GEMM_EX || r.kind == Kind::Q8ACT_GEMM)) {
+        c.ex = c.qg = false;
+        r = plan_route(c);
+        rc = ensure_ws(c.ctx, head + std::max(r.scratch, tail));
+    }
+    return rc;
+}
+
 // Validate, plan and launch one call with the context workspace as scratch.
-int run_matmul(const Call& c) {
+int run_matmul(Call c) {
     int rc = check_call(c);
     if (rc || c.m == 0) return rc;
     if (c.am) c.am->nb = 0;
@@ -961,21 +975,11 @@ int run_matmul(const Call& c) {
     if (r.kind == Kind::GEMM_EX) {
         const SideScratch side(c.ctx, c.s, r.scratch);
         if (side.p) return exec_route(c, r, side.p);
-        Call d = c;
-        d.ex = false;
-        r = plan_route(d);
+        c.ex = false;
+        r = plan_route(c);
     }
-    if (r.scratch) {
-        rc = ensure_ws(c.ctx, r.scratch);
-        if (rc && r.kind == Kind::Q8ACT_GEMM) {
-            // no room for its split sums: the row-tile kernels need the planes alone
-            Call d = c;
-            d.qg = false;
-            r = plan_route(d);
-            rc = ensure_ws(c.ctx, r.scratch);
-        }
-        if (rc) return rc;
-    }
+    rc = ensure_route(c, r);
+    if (rc) return rc;
     uint32_t* cnt = nullptr;
     if ((r.kind == Kind::GEMV_TILE || r.kind == Kind::Q8ACT_TILE) && r.tp.splits > 1 && tickets_on())
         cnt = tile_counters(c.ctx, (c.w->N + 31) / 32);  // >= output tiles
@@ -1678,10 +1682,10 @@ int thq_matmul_topk(thq_ctx* ctx, const thq_weight* w, const void* x_dev, thq_ac
     DeviceGuard g(ctx->device);
     // logits (workspace head unless the caller gives a buffer), then the
     // route's scratch and the top-k candidates, reserved in one step
-    const Route r = plan_route(c);
+    Route r = plan_route(c);
     const size_t lbytes = logits_dev ? 0 : round256((size_t)m * (size_t)w->N * sizeof(float));
     std::lock_guard<std::mutex> lk(ctx->mu);
-    rc = ensure_ws(ctx, lbytes + std::max(r.scratch, thq::topk_workspace_bytes(m, w->N, k)));
+    rc = ensure_route(c, r, lbytes, thq::topk_workspace_bytes(m, w->N, k));
     if (rc) return rc;
     float* logits = logits_dev ? logits_dev : static_cast<float*>(ctx->ws);
     void* scratch = static_cast<char*>(ctx->ws) + lbytes;
@@ -1743,10 +1747,10 @@ int thq_matmul_argmax(thq_ctx* ctx, const thq_weight* w, const void* x_dev, thq_
     // argmax scratch follow them: one reservation, sized from the route the
     // call will take, before any pointer into the workspace is formed
     c.am = nullptr;
-    const Route r = plan_route(c);
+    Route r = plan_route(c);
     const size_t lbytes = logits_dev ? 0 : round256((size_t)m * (size_t)w->N * sizeof(float));
     std::lock_guard<std::mutex> lk(ctx->mu);
-    rc = ensure_ws(ctx, lbytes + std::max(r.scratch, thq::argmax_workspace_bytes(m, w->N)));
+    rc = ensure_route(c, r, lbytes, thq::argmax_workspace_bytes(m, w->N));
     if (rc) return rc;
     float* logits = logits_dev ? logits_dev : static_cast<float*>(ctx->ws);
     void* scratch = static_cast<char*>(ctx->ws) + lbytes;
