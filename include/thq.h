@@ -26,17 +26,18 @@
  *    arrives; the buffer it outgrew stays allocated until thq_destroy, so
  *    work already enqueued, or captured in a HIP graph, keeps valid memory.
  *    A call that grows the workspace cannot run under stream capture: warm
- *    every captured shape once beforehand.  Calls on f32 rows do not use the
- *    shared workspace: they (and the split sums of thq_matmul_q8act from 9 rows)
- *    take scratch of their own from the context, so they stay re-entrant on
- *    distinct streams: a buffer per stream, grown like the workspace; past 16
- *    streams a stream takes over another's and waits for its work.  Captured
- *    ones need no warm-up for it: each captured graph gets scratch of its own
- *    (at most THQ_GRAPH_SCRATCH_MB, 4096, per context in all, kept until
- *    thq_destroy), so graphs may
- *    be replayed on any streams, beside each other and beside eager calls.
- *    Where none can be had (out of memory, the graphs' bound, eager calls on
- *    hipStreamPerThread) they run slower kernels that need none.
+ *    every captured shape once beforehand.  thq_matmul and
+ *    thq_gate_up_silu on f32 rows (outside THQ_MODE_Q8ACT) do not use the
+ *    shared workspace: they, and the split sums of thq_matmul_q8act and
+ *    thq_gate_up_silu_q8act[_emit] from 9 rows, take scratch of their own from
+ *    the context, so they stay re-entrant on distinct streams: a buffer per
+ *    stream, grown like the workspace; past 16 streams a stream takes over
+ *    another's and waits for its work.  Captured ones need no warm-up for it:
+ *    each captured graph gets scratch of its own (at most
+ *    THQ_GRAPH_SCRATCH_MB, 4096, per context in all, kept until thq_destroy),
+ *    so graphs may be replayed on any streams, beside each other and beside
+ *    eager calls.  Where none can be had (out of memory, the graphs' bound,
+ *    eager calls on hipStreamPerThread) they run slower kernels that need none.
  *  - W is [N, K] row-major (row n = output feature n), exactly the GGUF
  *    tensor layout QTensor::data() returns.  y[m, n] = sum_k x[m, k] * W[n, k].
  */
@@ -217,8 +218,9 @@ int thq_quantize_act(thq_ctx* ctx, thq_dtype dot_type, const void* x_dev, thq_ac
  * thq_matmul_q8act / thq_gate_up_silu_q8act consume it for any number of
  * weights whose dot type it is (THQ_Q8_0 for Q8_0 weights, THQ_Q8_K for
  * Q4_K) and whose K is k.  Results are bit-identical to thq_matmul /
- * thq_gate_up_silu with THQ_MODE_Q8ACT on the same x.  Returns 0 for an
- * unsupported dot type. */
+ * thq_gate_up_silu with THQ_MODE_Q8ACT on the same x, except that from 9 rows
+ * a call that finds no scratch (see Workspace above) sums the same exact block
+ * integers in another f32 order.  Returns 0 for an unsupported dot type. */
 size_t thq_q8act_bytes(thq_dtype dot_type, int64_t m, int64_t k);
 int thq_q8act_prepare(thq_ctx* ctx, thq_dtype dot_type, const void* x_dev, thq_act x_type, int64_t m, int64_t k,
                       void* buf_dev, void* stream);
@@ -239,8 +241,9 @@ int thq_gate_up_silu_q8act(thq_ctx* ctx, const thq_weight* fused, thq_dtype dot_
  * buffer the context owns (allocated and zeroed on the first call of a
  * larger shape; each launch leaves it zero), so such calls on one context
  * must be ordered on one stream.  A weight with a tile plane
- * (thq_weight_add_tiles) at 2..8 rows instead runs its int8 tile kernel and
- * then quantizes y in a second launch: the same bytes, faster there. */
+ * (thq_weight_add_tiles) at 2..8 rows instead runs its int8 tile kernel, and
+ * any weight from 9 rows by size the int8 matrix-core GEMM, and then quantizes
+ * y in a launch of its own: the same bytes, faster there, no counters. */
 int thq_gate_up_silu_q8act_emit(thq_ctx* ctx, const thq_weight* fused, thq_dtype dot_type, const void* buf_dev,
                                 int64_t m, int64_t k, void* y_dev, thq_act y_type, void* next_buf_dev,
                                 void* stream);

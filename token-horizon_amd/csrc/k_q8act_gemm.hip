@@ -26,9 +26,12 @@
 // rows go into LDS by direct-to-LDS copies, the next chunk's while the
 // current one computes.  A lane's 16 nibble bytes are its MFMA operand's 16
 // weights, so the conversion is one mask and two v_pk_mul_lo_u16 per 4
-// weights.  Bound: VALU (conversion and the f32 step) and MFMA together (a
-// chunk of gate/up at MH = 2 takes 2.75 us with one block on the CU, 5.4 with
-// two); weights by coalesced copies through LDS instead measured level.
+// weights.  Bound: no unit alone: gate/up of 24576 x 4096 at M = 256 (94 us)
+// keeps the VALU busy 38 % (conversion, the f32 step) and the matrix cores 24 %
+// of the time, 27 % of a wave's time in waits (a chunk at MH = 2 takes 2.75 us
+// with one block on the CU, 5.4 with two; Q4_K spills 2 to 3 registers there);
+// weights by coalesced copies through LDS instead measured slower (MLP at M =
+// 256: 180 against 169 us).
 #include "thq_dev.hpp"
 #include "thq_kernels.hpp"
 
