@@ -187,6 +187,25 @@ def test_capture_takes_the_eager_kernel():
             assert torch.equal(out, ref)
 
 
+def test_capture_without_scratch(monkeypatch):
+    """Past the bound on graph scratch a captured call runs the scalar kernel, which needs none."""
+    ctx = thq.Context(0)
+    w, x = weight("q4_k", 256, 1024, ctx), rows(5, 1024)
+    with monkeypatch.context() as mp:
+        mp.setenv("THQ_GEMM_EX", "0")
+        ref = thq.matmul(w, x, torch.float32)
+    monkeypatch.setenv("THQ_GRAPH_SCRATCH_MB", "0")
+    out = torch.empty_like(ref)
+    g = captured(w, x, out, torch.cuda.Stream())
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.randn(64, 64, device="cuda") @ torch.randn(64, 64, device="cuda")
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+
+
 def test_graphs_beside_each_other_and_eager_calls():
     """Graphs captured on one stream, replayed on others beside eager calls on that stream: every call's own bits."""
     w = weight("q4_k", 2048, 1024)

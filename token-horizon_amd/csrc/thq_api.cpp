@@ -265,7 +265,7 @@ void* graph_scratch(thq_ctx* ctx, hipStream_t s, unsigned long long id, size_t b
     for (const thq_graph_side& e : ctx->graph_side)
         if (e.id == id && e.s == s && e.bytes >= bytes) return e.p;
     const char* mb = getenv("THQ_GRAPH_SCRATCH_MB");
-    const size_t most = (size_t)(mb && *mb ? std::max(0l, atol(mb)) : GRAPH_SIDE_MB) << 20;
+    const size_t most = (size_t)(mb && *mb ? std::clamp(atol(mb), 0l, 1l << 30) : GRAPH_SIDE_MB) << 20;
     if (bytes > most || ctx->graph_side_bytes > most - bytes) return nullptr;
     try {
         ctx->graph_side.reserve(ctx->graph_side.size() + 1);
