@@ -350,7 +350,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
     constexpr float DOWN = 1.0f / EX_UP;
     __shared__ __attribute__((aligned(16))) uint8_t xs[2 * HB];
     __shared__ __attribute__((aligned(16))) float sas[NSUM ? 2 * NSUM * R : 1];
-    static_assert(2 * HB >= R * 64 * NW * 4, "the listed elements' products reuse xs");
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -684,32 +683,85 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
         return __builtin_fmaf(DOWN, acc[t][0][(e + 4) & 15] + acc[t][0][(e + 8) & 15], acc[t][0][e]);
     };
     constexpr int NT = GU && OUT != 0 ? 1 : 2;  // stored tiles (gate/up: one, the gate's)
-    // the rows with listed elements, and of those the ones dotted whole: f32
-    // dots over the split's K into LDS (lane half g takes every other element)
+    // The rows with listed elements, and of those the ones dotted whole: f32
+    // dots over the split's K, summed in LDS (xs, no copy is in flight).  Here a
+    // lane has one weight row, that of tile g.  The group's listed elements
+    // that lie in the split are gathered first, row after row, so that the
+    // loads of eight of them are in flight together (one row after the other
+    // took 4 times as long as the GEMM at M = 300 with eight in each row).
     const int lc = lane < Mz ? LC[m0 + lane] : 0;
     const uint32_t some = (uint32_t)__ballot(lc != 0), whole = (uint32_t)__ballot(lc < 0);
-    float* const side = reinterpret_cast<float*>(xs) + wave * 64 + n;  // [row][wave][t][n], no copy in flight
-    for (uint32_t left = some; left; left &= left - 1) {
-        const int m = __builtin_ctz(left);
-        const bool all = (whole >> m) & 1;
-        const int cnt = all ? (ce - cb) * 256 : __builtin_amdgcn_readlane(lc, m);
-        float v[2] = {0.0f, 0.0f};
-#pragma clang loop unroll(disable)
-        for (int i = g; i < cnt; i += 2) {
+    constexpr int COLS = 64 * NW;
+    float* const side = reinterpret_cast<float*>(xs);  // [row][wave][tile][n]
+    if (some) {
+        struct Flat {
+            int m;
             ExItem it;
-            if (all) {
-                it.k = cb * 256 + i;
-                it.x = load_x<float>(X + (int64_t)(m0 + m) * K + it.k);
-            } else {
-                it = LK[(int64_t)(m0 + m) * EX_LIST + i];
-                if (it.k < cb * 256 || it.k >= ce * 256) continue;
-            }
+        };
+        Flat* const flat = reinterpret_cast<Flat*>(side + R * COLS);
+        int* const counts = reinterpret_cast<int*>(flat + R * EX_LIST);
+        static_assert(2 * HB >= R * COLS * 4 + R * EX_LIST * (int)sizeof(Flat) + R * 4, "all of it in xs");
+        constexpr int PER = EX_LIST / 8;  // a row's elements over eight threads
+        const int64_t rw = row[g];
+        float* const own = side + wave * 64 + lane;
+        for (uint32_t left = some; left; left &= left - 1) own[__builtin_ctz(left) * COLS] = 0.0f;
+        const int tm = (int)threadIdx.x >> 3, ti = (int)threadIdx.x & 7;
+        const int tn = tm < Mz ? LC[m0 + tm] : 0;
+        ExItem it[PER];
+        int found = 0;  // in the split, and (upper half) before it
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
-                v[t] = __builtin_fmaf(it.x, ex_weight<QT>(Wq, Wa, row[t], K, nrows, it.k), v[t]);
+        for (int q = 0; q < PER; ++q) {
+            it[q].k = -1;
+            if (ti + 8 * q >= tn) continue;
+            it[q] = LK[(int64_t)(m0 + tm) * EX_LIST + ti + 8 * q];
+            found += it[q].k < cb * 256 ? 1 << 16 : it[q].k < ce * 256 ? 1 : 0;
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) side[m * 64 * NW + 32 * t] = v[t] + __shfl_xor(v[t], 32, 64);
+        for (int off = 1; off < 8; off <<= 1) found += __shfl_xor(found, off, 64);
+        if (ti == 0 && tm < R) counts[tm] = found & 0xFFFF;
+        __syncthreads();
+        int total = 0, base = 0;
+        for (int i = 0; i < R; ++i) {
+            base = i == tm ? total : base;
+            total += counts[i];
+        }
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+            if (it[q].k >= cb * 256 && it[q].k < ce * 256) flat[base + ti + 8 * q - (found >> 16)] = Flat{tm, it[q]};
+        __syncthreads();
+        for (int i = 0; i < total; i += 8) {
+            Flat f[8];
+            float w[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = flat[i + j < total ? i + j : i];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) w[j] = ex_weight<QT>(Wq, Wa, rw, K, nrows, f[j].it.k);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (i + j < total) own[f[j].m * COLS] = __builtin_fmaf(f[j].it.x, w[j], own[f[j].m * COLS]);
+        }
+        if (whole) {
+            for (int k = cb * 256; k < ce * 256; k += 32) {  // the weights once for all those rows
+                float w[32];
+#pragma unroll
+                for (int i = 0; i < 32; ++i) w[i] = ex_weight<QT>(Wq, Wa, rw, K, nrows, k + i);
+                for (uint32_t left = whole; left; left &= left - 1) {
+                    const int m = __builtin_ctz(left);
+                    const float4* x = reinterpret_cast<const float4*>(X + (int64_t)(m0 + m) * K + k);
+                    float v = own[m * COLS];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float4 q = x[i];
+                        v = __builtin_fmaf(q.x, w[4 * i], v);
+                        v = __builtin_fmaf(q.y, w[4 * i + 1], v);
+                        v = __builtin_fmaf(q.z, w[4 * i + 2], v);
+                        v = __builtin_fmaf(q.w, w[4 * i + 3], v);
+                    }
+                    own[m * COLS] = v;
+                }
+            }
+        }
+        __syncthreads();
     }
 #pragma unroll
     for (int e = 0; e < R / 2; ++e) {
@@ -722,7 +774,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_ex(const uint8_t* Wq, const uin
         if ((some >> m) & 1) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const float f = side[m * 64 * NW + 32 * t];
+                const float f = side[m * COLS + wave * 64 + 32 * t + n];
                 v[t] = (whole >> m) & 1 ? f : v[t] + f;
             }
         }
