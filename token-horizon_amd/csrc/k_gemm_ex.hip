@@ -922,8 +922,10 @@ ExPlan plan_gemm_ex(int qtype, int64_t M, int64_t N, int64_t K, bool gu, int cus
                                                      : (uint64_t)((N + 3) / 4) * (uint64_t)(K / 256) * 576u);
     if (plane >= lim || (uint64_t)M * (uint64_t)K * 6u >= lim) return p;
     // Two blocks per CU.  Cost of a K split count: rounds of resident blocks
-    // x chunks (and one of prologue) x a chunk's time (2.4 us stacked, 4.0 us
-    // with 32 rows), plus the partials' round trip at 4 TB/s.
+    // x chunks (and one of prologue) x a chunk's weight (2.4 us stacked, 4.0 us
+    // with 32 rows: less than a chunk takes with both blocks there, but dearer
+    // chunks, 3.0 and 8.0, plan more splits at 300 rows: the 4096 / 12288 MLP 487
+    // against 465 us), plus the partials' round trip at 4 TB/s.
     const int64_t nch = K / 256, nout = gu ? N / 2 : N, cu = cus > 0 ? cus : 256;
     p.rows = M <= 8 ? 8 : M <= 16 ? 16 : 32;
     p.groups = (int)((M + p.rows - 1) / p.rows);

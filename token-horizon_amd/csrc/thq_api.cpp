@@ -549,9 +549,10 @@ thq::QgRows q8act_gemm_plan(const thq_ctx* ctx, const thq_weight* w, int64_t m, 
 // f32 rows: k_gemm_ex (every format, K in whole chunks) in row chunks whose
 // scratch (activation planes, split partials) stays within EX_MAX_MB and the
 // caller's cap, where the scalar generic kernel ran before and the call is
-// large enough for its three launches (scalar / it, us: 2 rows of 3072 x 1024
-// 10.9 / 16.0, 2 rows of 4096 x 4096 Q4_K 17.6 / 17.1, Q6_K 18.7 / 21.6; 5 rows
-// 40.8 / 17.8, 41.8 / 21.9).  THQ_GEMM_EX: 0 never, 1 wherever supported
+// large enough for its three launches (scalar / it, us: 3072 x 1024 at 2 / 5 / 8
+// rows 6.2 / 11.6 / 17.3 against 12.6 / 13.2 / 13.3, 4096 x 4096 at 2 / 3 / 8 rows
+// Q4_K 17.5 / 24.7 / 60.3 against 14.8 / 15.1 / 15.7, Q6_K 18.1 / 25.2 / 61.0
+// against 18.7 / 18.9 / 19.6).  THQ_GEMM_EX: 0 never, 1 wherever supported
 // (tests), unset: that rule.
 constexpr size_t EX_MAX_MB = 512;
 bool plan_ex(const Call& c, Route& r) {
